@@ -1624,9 +1624,10 @@ int load_mode_for(const GemmArgs &a, bool ta, bool tb, int bm, int bn) {
 
 template <typename T, bool TA, bool TB, bool DUAL>
 hipError_t launch_cfg(const TileCfg &cfg, const GemmArgs &a, dim3 grid, hipStream_t s) {
-    const int mode = DUAL ? (tiles_exact(a, cfg.bm, cfg.bn / 2, ET<T>::BK) ? LOAD_EXACT
-                             : vectors_exact<T>(a, TA, TB)                  ? LOAD_MASKED
-                                                                            : LOAD_CHECKED)
+    // cfg.bn is the output tile's width: for SwiGLU already half of the B tile's rows.
+    const int mode = DUAL ? (tiles_exact(a, cfg.bm, cfg.bn, ET<T>::BK) ? LOAD_EXACT
+                             : vectors_exact<T>(a, TA, TB)              ? LOAD_MASKED
+                                                                        : LOAD_CHECKED)
                           : load_mode_for<T>(a, TA, TB, cfg.bm, cfg.bn);
     if (mode == LOAD_EXACT)
         launch_cfg_lm<T, TA, TB, DUAL, LOAD_EXACT>(cfg, a, grid, s);
