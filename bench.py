@@ -36,7 +36,8 @@ import numpy as np
 ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
-PEAK_TFLOPS = {"f32": 157.3, "bf16": 2500.0}
+# FP32 products run as six BF16 products each (the FP32 units reach 157.3).
+PEAK_TFLOPS = {"f32": 2500.0 / 6, "bf16": 2500.0}
 PEAK_HBM_GBS = 8000.0
 
 

@@ -32,6 +32,7 @@ IT_EPI_CAUSAL = 0x4
 IT_EPI_ROPE = 0x8
 IT_EPI_SWIGLU_BWD = 0x10
 IT_EPI_XENT_A = 0x20
+IT_EPI_F32_UNITS = 0x40
 
 c_void_p = C.c_void_p
 c_i64 = C.c_int64

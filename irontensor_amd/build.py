@@ -5,7 +5,7 @@ The compile always runs; objects go to irontensor_amd/_build/ and the shared lib
 file, so it travels with the repository snapshot to the GPU box.
 
 python -m irontensor_amd.build --tuning also builds libirontensor_hip_tuning.so: the same library
-with kernels_gemm.hip compiled under IT_TUNING, where the environment variable IT_PLAN="tile,
+with the GEMM sources compiled under IT_TUNING, where the environment variable IT_PLAN="tile,
 splits[,width]" forces every GEMM's plan and IT_GROUP_SPLITS an FP32 group's split count (planner
 measurements only: load it with IRONTENSOR_LIB=...; nothing else uses it).
 """
@@ -24,9 +24,10 @@ LIB = PKG / "libirontensor_hip.so"
 TUNING_LIB = PKG / "libirontensor_hip_tuning.so"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["runtime.cpp", "api.cpp", "api_train.cpp", "kernels_gemm.hip", "kernels_misc.hip", "kernels_flash.hip",
-           "kernels_gemv.hip", "kernels_train.hip", "noalloc.hip",
-           "kernels_flash2.hip"]
+SOURCES = ["runtime.cpp", "api.cpp", "api_train.cpp", "kernels_gemm.hip", "kernels_gemm_f32.hip", "kernels_misc.hip",
+           "kernels_flash.hip", "kernels_gemv.hip", "kernels_train.hip", "noalloc.hip", "kernels_flash2.hip"]
+#: Sources with planner overrides (IT_TUNING).
+TUNED = ["kernels_gemm.hip", "kernels_gemm_f32.hip"]
 
 # -packed-fp32-ops: hipcc must not emit packed FP32 ALU ops (v_pk_*_f32) on this pool.
 HIP_FLAGS = [
@@ -72,16 +73,18 @@ def build_library(verbose: bool = False) -> Path:
 
 
 def build_tuning_library() -> Path:
-    """The library with kernels_gemm.hip under IT_TUNING (plans forced through IT_PLAN), linked with
+    """The library with the GEMM sources under IT_TUNING (plans forced through IT_PLAN), linked with
     the other objects of the last build_library()."""
     tdir = BUILD / "tuning"
     tdir.mkdir(parents=True, exist_ok=True)
-    obj = tdir / "kernels_gemm.hip.o"
-    cmd = [HIPCC, *HIP_FLAGS, "-DIT_TUNING", "-x", "hip", "-c", str(CSRC / "kernels_gemm.hip"), "-o", str(obj)]
-    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed:\n{res.stdout}")
-    objs = [str(BUILD / (name + ".o")) for name in SOURCES if name != "kernels_gemm.hip"] + [str(obj)]
+    objs = [str(BUILD / (name + ".o")) for name in SOURCES if name not in TUNED]
+    for name in TUNED:
+        obj = tdir / (name + ".o")
+        cmd = [HIPCC, *HIP_FLAGS, "-DIT_TUNING", "-x", "hip", "-c", str(CSRC / name), "-o", str(obj)]
+        res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        if res.returncode != 0:
+            raise RuntimeError(f"hipcc failed:\n{res.stdout}")
+        objs.append(str(obj))
     tmp = TUNING_LIB.with_suffix(".so.tmp")
     res = subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *objs],
                          stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -68,31 +68,32 @@ it_status it_gemm_check(it_dtype dtype_in, it_dtype dtype_out, it_op transA, it_
     if (has_out && !C) return fail(IT_ERR_NULL, "matmul: C is NULL");
     if (has_out && K > 0 && (!A || !B)) return fail(IT_ERR_NULL, "matmul: A or B is NULL");
     if (epi) {
+        const uint32_t flags = epi->flags & ~IT_EPI_F32_UNITS;  // selects the kernels, combines with everything
         const uint32_t known =
             IT_EPI_BIAS | IT_EPI_SWIGLU | IT_EPI_CAUSAL | IT_EPI_ROPE | IT_EPI_SWIGLU_BWD | IT_EPI_XENT_A;
-        if (epi->flags & ~known) return fail(IT_ERR_INVALID, "matmul: unknown epilogue flags");
-        if ((epi->flags & IT_EPI_BIAS) && !epi->bias)
+        if (flags & ~known) return fail(IT_ERR_INVALID, "matmul: unknown epilogue flags");
+        if ((flags & IT_EPI_BIAS) && !epi->bias)
             return fail(IT_ERR_NULL, "matmul: bias epilogue without a bias pointer");
-        if (epi->flags & IT_EPI_SWIGLU) {
+        if (flags & IT_EPI_SWIGLU) {
             if (!epi->B2 && has_out && K > 0)
                 return fail(IT_ERR_NULL, "matmul: SwiGLU epilogue without B2");
             if (transA != IT_OP_N || transB != IT_OP_T)
                 return fail(IT_ERR_INVALID, "matmul: SwiGLU epilogue needs transA=N, transB=T (Y = X.W^T)");
-            if (epi->flags & IT_EPI_CAUSAL)
+            if (flags & IT_EPI_CAUSAL)
                 return fail(IT_ERR_INVALID, "matmul: SwiGLU epilogue cannot be combined with causal");
         }
-        if ((epi->flags & (IT_EPI_SWIGLU | IT_EPI_CAUSAL)) && beta != 0.f)
+        if ((flags & (IT_EPI_SWIGLU | IT_EPI_CAUSAL)) && beta != 0.f)
             return fail(IT_ERR_INVALID, "matmul: beta != 0 cannot be combined with SwiGLU or causal");
-        if (epi->flags & IT_EPI_SWIGLU_BWD) {
-            if (epi->flags != IT_EPI_SWIGLU_BWD)
+        if (flags & IT_EPI_SWIGLU_BWD) {
+            if (flags != IT_EPI_SWIGLU_BWD)
                 return fail(IT_ERR_INVALID, "matmul: the SwiGLU-backward epilogue combines with no other flag");
             if (beta != 0.f) return fail(IT_ERR_INVALID, "matmul: beta != 0 cannot be combined with SwiGLU backward");
             if (has_out && (!epi->gate_out || !epi->up_out))
                 return fail(IT_ERR_NULL, "matmul: SwiGLU-backward epilogue without gate or up");
             if (batch > 1) return fail(IT_ERR_INVALID, "matmul: SwiGLU backward is a single (unbatched) product");
         }
-        if (epi->flags & IT_EPI_XENT_A) {
-            if (epi->flags != IT_EPI_XENT_A)
+        if (flags & IT_EPI_XENT_A) {
+            if (flags != IT_EPI_XENT_A)
                 return fail(IT_ERR_INVALID, "matmul: the cross-entropy operand combines with no other flag");
             if (dtype_in != IT_F32)
                 return fail(IT_ERR_PRECISION, "matmul: the cross-entropy operand needs FP32 inputs");
@@ -103,8 +104,8 @@ it_status it_gemm_check(it_dtype dtype_in, it_dtype dtype_out, it_op transA, it_
             if ((uintptr_t)epi->xent_stats % 8 != 0)
                 return fail(IT_ERR_INVALID, "matmul: cross-entropy stats must be 8-byte aligned");
         }
-        if (epi->flags & IT_EPI_ROPE) {
-            if (epi->flags & (IT_EPI_SWIGLU | IT_EPI_CAUSAL))
+        if (flags & IT_EPI_ROPE) {
+            if (flags & (IT_EPI_SWIGLU | IT_EPI_CAUSAL))
                 return fail(IT_ERR_INVALID, "matmul: RoPE cannot be combined with SwiGLU or causal");
             if (epi->rope_head_dim <= 0 || epi->rope_head_dim % 2 != 0 || epi->rope_seq <= 0 ||
                 epi->rope_cols < 0 || epi->rope_cols > N || epi->rope_cols % epi->rope_head_dim != 0 ||
@@ -145,6 +146,7 @@ static it_status gemm_args(it_context *ctx, it_dtype dtype_in, it_dtype dtype_ou
     a.b_vec_ok = vec_ok(B, eb, ldb, strideB, 0);
     a.c_vec_ok = out_vec_ok(C, a.out_bf16, ldc, strideC, 0);
     if (epi) {
+        a.f32_units = (epi->flags & IT_EPI_F32_UNITS) != 0;
         a.has_bias = (epi->flags & IT_EPI_BIAS) != 0;
         a.bias = epi->bias;
         if (epi->flags & IT_EPI_SWIGLU) {

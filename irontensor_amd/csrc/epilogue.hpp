@@ -11,6 +11,9 @@
 namespace it {
 namespace {
 
+// Four FP32 values of an output row: 128-bit accesses that need an element's alignment only.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 __device__ __forceinline__ float load_out(const void *C, int64_t idx, int bf16) {
     return bf16 ? bf16_to_f32(((const uint16_t *)C)[idx]) : ((const float *)C)[idx];
 }
@@ -81,8 +84,8 @@ __device__ __forceinline__ void finish4(const GemmArgs &p, f32x4 v, int64_t row,
                 u = f32x4{__uint_as_float(uh[0] << 16), __uint_as_float(uh[0] & 0xffff0000u),
                           __uint_as_float(uh[1] << 16), __uint_as_float(uh[1] & 0xffff0000u)};
             } else {
-                g = *(const f32x4 *)((const float *)p.G + gi);
-                u = *(const f32x4 *)((const float *)p.U + gi);
+                g = *(const f32x4_any *)((const float *)p.G + gi);
+                u = *(const f32x4_any *)((const float *)p.U + gi);
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -94,8 +97,8 @@ __device__ __forceinline__ void finish4(const GemmArgs &p, f32x4 v, int64_t row,
                 *(u32x2 *)((uint16_t *)p.C + idx) = u32x2{pack_bf16x2(dg[0], dg[1]), pack_bf16x2(dg[2], dg[3])};
                 *(u32x2 *)((uint16_t *)p.C + idx + p.N) = u32x2{pack_bf16x2(du[0], du[1]), pack_bf16x2(du[2], du[3])};
             } else {
-                *(f32x4 *)((float *)p.C + idx) = dg;
-                *(f32x4 *)((float *)p.C + idx + p.N) = du;
+                *(f32x4_any *)((float *)p.C + idx) = dg;
+                *(f32x4_any *)((float *)p.C + idx + p.N) = du;
             }
             return;
         }
@@ -107,7 +110,7 @@ __device__ __forceinline__ void finish4(const GemmArgs &p, f32x4 v, int64_t row,
                 old = f32x4{__uint_as_float(o[0] << 16), __uint_as_float(o[0] & 0xffff0000u),
                             __uint_as_float(o[1] << 16), __uint_as_float(o[1] & 0xffff0000u)};
             } else {
-                old = *(const f32x4 *)((const float *)p.C + idx);
+                old = *(const f32x4_any *)((const float *)p.C + idx);
             }
             v += p.beta * old;
         }
@@ -138,7 +141,7 @@ __device__ __forceinline__ void finish4(const GemmArgs &p, f32x4 v, int64_t row,
             o[1] = pack_bf16x2(v[2], v[3]);
             *(u32x2 *)((uint16_t *)p.C + idx) = o;
         } else {
-            *(f32x4 *)((float *)p.C + idx) = v;
+            *(f32x4_any *)((float *)p.C + idx) = v;
         }
         return;
     }
@@ -177,9 +180,9 @@ __device__ __forceinline__ void finish_swiglu4(const GemmArgs &p, f32x4 g, f32x4
             if (p.U) st(p.U, u);
             st(p.C, h);
         } else {
-            if (p.G) *(f32x4 *)((float *)p.G + idx) = g;
-            if (p.U) *(f32x4 *)((float *)p.U + idx) = u;
-            *(f32x4 *)((float *)p.C + idx) = h;
+            if (p.G) *(f32x4_any *)((float *)p.G + idx) = g;
+            if (p.U) *(f32x4_any *)((float *)p.U + idx) = u;
+            *(f32x4_any *)((float *)p.C + idx) = h;
         }
         return;
     }

@@ -148,6 +148,7 @@ struct GemmArgs {
     const float *row_scale;
     float rms_eps;
     int no_split;  // the planner must not split K
+    int f32_units;  // FP32: sums on the FP32 units, in k order (IT_EPI_F32_UNITS)
     // RoPE on the result (epilogue, 4-column vectors): columns < rope_cols rotate pairwise (2i,
     // 2i+1 of each head of 2 rope_half columns) by rope_table[(row % rope_seq) * rope_half + i].
     const float2 *rope_table;
@@ -192,6 +193,14 @@ it_status launch_gemm(it_context *ctx, it_dtype dtype_in, bool transA, bool tran
 // where they pay (kernels_gemm.hip), else launch_gemm for each.
 it_status launch_gemm_group(it_context *ctx, it_dtype dtype_in, const bool *ta, const bool *tb, GemmArgs *args,
                             int count, const char *profile_tag);
+
+// FP32 products as BF16 terms (kernels_gemm_f32.hip): every product without an operand transform whose
+// operands fit 31-bit offsets, unless the caller asks for the FP32 units.
+bool f32_terms_applicable(const GemmArgs &a, bool ta, bool tb);
+it_status launch_gemm_f32(it_context *ctx, bool transA, bool transB, GemmArgs args, const char *profile_tag);
+// Products of one layout as one launch where it pays; false (nothing launched) where it does not.
+bool launch_gemm_f32_group(it_context *ctx, bool ta, bool tb, const GemmArgs *args, int count, const char *profile_tag,
+                           it_status *status);
 
 // Fused attention (kernels_flash.hip), head_dim 64. Per-head addressing of each operand:
 // (bh / heads) * bs + (bh % heads) * hs + row * rs + col (element strides).

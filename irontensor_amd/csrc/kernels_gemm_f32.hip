@@ -1,0 +1,826 @@
+// FP32 GEMMs on the BF16 matrix units: every operand element is split into three BF16 terms on its way
+// into LDS (split_bf16x3: 24 significand bits), and a product takes the six term products down to
+// 2^-16 of the whole, accumulated in FP32. The FP32 units reach 157 TFLOP/s; six BF16 products per
+// FP32 product 417 at the nominal BF16 rate and 228 at the rate the largest BF16 products reach on
+// this card.
+//
+// Design (per k-tile of 32):
+//   * global -> registers with 128-bit buffer loads (k-contiguous operands: 4 k of a row; mn-contiguous
+//     ones: 2 or 4 k-rows x 4 columns, so that the split, which packs pairs of k, transposes on the
+//     way). A descriptor ends at the operand's last element and its range check, dword by dword,
+//     supplies the zeros past it; the loads need no more than an element's alignment. So every size
+//     and leading dimension runs the same loop (a 1000 x 300 x 701 layer forward and backward: 53 us
+//     with the FP32-unit kernels, whose loads go element by element there, 46 here);
+//   * split, then three LDS planes [rows][32 k] of 64-byte rows; a lane's fragment of one term is one
+//     128-bit LDS read;
+//   * v_mfma_f32_16x16x32_bf16 blocks (the 32x32x16 form measured 2-6% slower in these tiles);
+//   * one LDS stage and two barriers per k-tile (gemm_f32_block), so that several blocks share a CU;
+//   * an accumulator that is not finite is computed again on the FP32 units, since the terms of an
+//     infinity (or of a value that rounds up to 2^128) are NaN.
+#include <cstdio>
+#include <string>
+
+#include "gemm_tiles.hpp"
+
+namespace it {
+namespace {
+
+// One operand's k-tile: global -> registers -> LDS terms, and LDS -> MFMA fragments.
+//   KCONTIG: global element (r, k) at base[r * ld + k] (A not transposed, or B transposed).
+//   otherwise: global element (r, k) at base[k * ld + r].
+template <bool KCONTIG_, int ROWS, int THREADS>
+struct F32Operand {
+    static constexpr bool KCONTIG = KCONTIG_;
+    static constexpr int NT = THREADS;
+    static constexpr int VEC = 4, BK = ET<float>::BK;
+    static constexpr int PLANE = ROWS * 64;  // bytes of one term's plane
+    static constexpr int STAGE_BYTES = 3 * PLANE;
+    // k-rows of an mn-contiguous unit: 2 where 4 would leave threads without a unit.
+    static constexpr int KQ = (BK / 4) * (ROWS / VEC) < THREADS ? 2 : 4;
+    static constexpr int KGROUPS = BK / KQ;
+    static constexpr int LOADS = KCONTIG ? 1 : KQ;
+    static constexpr int ITEMS = KCONTIG ? ROWS * BK / VEC : KGROUPS * (ROWS / VEC);
+    static constexpr int ITERS = (ITEMS + THREADS - 1) / THREADS;
+
+    u32x4 reg[ITERS][LOADS];
+
+    // mn-contiguous units: (k-group of KQ rows, 4 columns), the k-groups fastest.
+    __device__ __forceinline__ static void unit(int item, int &kg, int &rc) {
+        kg = item % KGROUPS;
+        rc = item / KGROUPS;
+    }
+
+    // Byte of k position kb / 2 (kb: byte in the 64-byte row) of `row` in a plane. Rows swap places
+    // within groups of 4 by the group's number, and a row's 16-byte chunks by its place: measured, a
+    // fragment's 128-bit reads (16 rows, 4 chunks) then go at 203 bytes per clock and CU, as linear
+    // ones do (122 without the chunk swap), and every write pattern (8 bytes of consecutive rows or
+    // of rows 4 apart, 4 bytes of rows 4 apart) at its linear rate (65, 50).
+    __device__ __forceinline__ static int off(int row, int kb) {
+        const int q = (row & ~3) | ((row ^ (row >> 2)) & 3);
+        return q * 64 + ((((kb >> 4) ^ (q >> 1)) & 3) << 4) + (kb & 15);
+    }
+
+    // Zeros the elements of a k-contiguous tile at k positions from `left` on (its row's next
+    // elements, or the next row's).
+    __device__ __forceinline__ void mask(int64_t left, int tid) {
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            const int kc = (tid + it * THREADS) % (BK / VEC);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) reg[it][0][e] = kc * VEC + e < left ? reg[it][0][e] : 0u;
+        }
+    }
+
+    // Splits and writes part `part` of `parts` of the tile (the caller interleaves them with MFMAs).
+    __device__ __forceinline__ void store(char *lds, int tid, int part, int parts) const {
+        constexpr int PIECES = KCONTIG ? ITERS : 4 * ITERS;
+        auto mine = [&](int piece) { return piece * parts / PIECES == part; };
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            const int item = tid + it * THREADS;
+            if (ITEMS % THREADS != 0 && item >= ITEMS) continue;
+            if constexpr (KCONTIG) {
+                if (!mine(it)) continue;
+                const int rr = item / (BK / VEC), kc = item % (BK / VEC);
+                const u32x4 &v = reg[it][0];
+                const Bf16x3 a = split_bf16x3(v[0], v[1]), b = split_bf16x3(v[2], v[3]);
+                char *d = lds + off(rr, kc * 8);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) *(u32x2 *)(d + p * PLANE) = u32x2{a.t[p], b.t[p]};
+            } else {
+                int kg, rc;
+                unit(item, kg, rc);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (!mine(it * 4 + j)) continue;
+                    char *d = lds + off(rc * 4 + j, kg * KQ * 2);
+                    const Bf16x3 a = split_bf16x3(reg[it][0][j], reg[it][1][j]);
+                    if constexpr (KQ == 4) {
+                        const Bf16x3 b = split_bf16x3(reg[it][2][j], reg[it][3][j]);
+#pragma unroll
+                        for (int p = 0; p < 3; ++p) *(u32x2 *)(d + p * PLANE) = u32x2{a.t[p], b.t[p]};
+                    } else {
+#pragma unroll
+                        for (int p = 0; p < 3; ++p) *(uint32_t *)(d + p * PLANE) = a.t[p];
+                    }
+                }
+            }
+        }
+    }
+
+    // Term p of the v_mfma_f32_16x16x32_bf16 fragment of the 16 rows from `row` (a multiple of 16):
+    // lane l holds row l % 16 at k 8 (l / 16) .. +7.
+    __device__ __forceinline__ static u32x4 frag(const char *lds, int row, int p, int lane) {
+        return *(const u32x4 *)(lds + p * PLANE + row * 64 + off(lane & 15, (lane >> 4) * 16));
+    }
+};
+
+// The loads of an operand tile O: a descriptor from the tile's first element to the operand's last,
+// each item's byte offset, formed once per block, and the k-tile's as the load's scalar offset, so a
+// load costs no vector instruction besides itself. Past the end the range check returns zeros: rows
+// past M or N of a k-contiguous operand, k past K of an mn-contiguous one. An mn-contiguous operand's
+// columns past M (or N) read the next row's elements; they reach only outputs that are not stored.
+template <class O>
+struct TileLoad {
+    __amdgpu_buffer_rsrc_t rs;
+    uint32_t voff[O::ITERS][O::LOADS];
+    uint32_t kstride;
+
+    // base: the operand of this batch item, rows x K; r0: the tile's first row.
+    __device__ __forceinline__ void init(const float *base, int64_t ld, int64_t rows, int64_t K, int64_t r0, int tid) {
+        const int64_t skip = O::KCONTIG ? r0 * ld : r0;
+        const int64_t left = (O::KCONTIG ? (rows - 1) * ld + K : (K - 1) * ld + rows) - skip;
+        const int n = left > 0x1fffffff ? 0x7fffffff : (int)(left * 4);
+        rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base + skip), (short)0, n, 0x00020000);
+        kstride = O::KCONTIG ? 4u : (uint32_t)(ld * 4);
+#pragma unroll
+        for (int it = 0; it < O::ITERS; ++it) {
+            const int item = tid + it * O::NT;
+            if constexpr (O::KCONTIG) {
+                const int rr = item / (O::BK / O::VEC), kc = item % (O::BK / O::VEC);
+                voff[it][0] = (uint32_t)((rr * ld + kc * O::VEC) * 4);
+            } else {
+                int kg, rc;
+                O::unit(item, kg, rc);
+#pragma unroll
+                for (int q = 0; q < O::LOADS; ++q)
+                    voff[it][q] = (uint32_t)(((kg * O::KQ + q) * ld + rc * O::VEC) * 4);
+            }
+        }
+    }
+
+    __device__ __forceinline__ void load(O &o, int64_t k0, int tid) const {
+        const uint32_t koff = (uint32_t)k0 * kstride;
+#pragma unroll
+        for (int it = 0; it < O::ITERS; ++it) {
+            const int item = tid + it * O::NT;
+            if (O::ITEMS % O::NT != 0 && item >= O::ITEMS) continue;
+#pragma unroll
+            for (int q = 0; q < O::LOADS; ++q)
+                o.reg[it][q] =
+                    __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff[it][q], koff, 0));
+        }
+    }
+};
+
+// Byte offsets from a tile's start within 31 bits: a k-contiguous operand's rows, or an mn-contiguous
+// one's k range (with the k-tile past its end that a block reads ahead).
+bool spans_fit(const GemmArgs &a, bool ta, bool tb) {
+    auto fits = [&](bool kcontig, int64_t ld) { return (kcontig ? 256 * ld + a.K : (a.K + 64) * ld) * 4 < (1ll << 31); };
+    return fits(!ta, a.lda) && fits(tb, a.ldb);
+}
+
+// The tile shapes: BM x BN output tiles of WM x WN waves, times KG groups of them, each with its own
+// LDS stage, that take every KG-th k-tile (group 0 adds the others' sums and finishes the tile).
+template <int BM_, int BN_, int WM_, int WN_, int KG_ = 1>
+struct Shape {
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, KG = KG_;
+    static constexpr int THREADS = WM * WN * 64;  // of one k group
+    static constexpr bool WIDE = BM * BN / (WM * WN) >= 64 * 64;
+    // Waves per SIMD the registers are held to.
+    static constexpr int WAVES = WIDE ? 2 : KG > 1 ? 4 : 3;
+    static constexpr int SMEM = 3 * 64 * (BM + BN);
+};
+using S128 = Shape<128, 128, 2, 2>;      // 64 x 64 per wave, two blocks per CU
+using S256 = Shape<256, 128, 4, 2>;      // the same per wave, one block per CU
+using S64 = Shape<64, 64, 2, 2>;         // 32 x 32 per wave, three blocks per CU
+using S6432 = Shape<64, 32, 2, 2, 2>;    // 32 x 16 per wave, two blocks of eight waves per CU
+
+// One block: output tile `tile` (in map_tile order) of batch-and-split index z, with `smem0` of KG *
+// S::SMEM bytes.
+// DUAL: the B tile's rows 0..BN/2-1 are gate-weight rows and BN/2..BN-1 the same up-weight rows.
+// FIX (64 x 64 tiles of batch-1 products): with split K, each split's partial tile goes to p.partial
+// at device scope and the tile's last block to arrive at `arrive` (a zero counter, left at zero)
+// adds the splits in split order and runs the epilogue, so no separate reduction launch follows.
+template <class S, bool TA, bool TB, bool DUAL, bool FIX = false>
+__device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int64_t z, char *smem0,
+                                               int *arrive = nullptr) {
+    constexpr int BM = S::BM, BN = S::BN, WM = S::WM, WN = S::WN, KG = S::KG, THREADS = S::THREADS;
+    constexpr int BK = ET<float>::BK;
+    constexpr int WTM = BM / WM, WTN = BN / WN, FM = WTM / 16, FN = WTN / 16;
+    static_assert(KG == 1 || (BM == 64 && !DUAL && !FIX), "k groups: plain products");
+    // Tiles of 64 rows store straight from transposed accumulators; larger ones stage the epilogue
+    // through LDS, whose full-line stores suit outputs of hundreds of megabytes; SwiGLU pairs waves
+    // in LDS.
+    constexpr bool XPOSE = !DUAL && BM == 64;
+    using OA = F32Operand<!TA, BM, THREADS>;
+    using OB = F32Operand<TB, BN, THREADS>;
+    using OBL = F32Operand<TB, DUAL ? BN / 2 : BN, THREADS>;  // as loaded (DUAL: the gate or up half)
+    static_assert(!DUAL || (!TA && TB), "SwiGLU is Y = X.W^T");
+    constexpr int SA = OA::STAGE_BYTES;
+
+    const int tid = threadIdx.x % THREADS, lane = tid & 63, wave = tid >> 6;
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / THREADS);
+    const int wm = wave / WN, wn = wave % WN;
+    char *const smem = KG == 1 ? smem0 : smem0 + kg * S::SMEM;
+    int tm, tn;
+    map_tile(tile, p.tiles_m, p.tiles_n, tm, tn);
+    const int64_t b = z % p.batch, split = z / p.batch;
+    const int64_t bo = b / p.batch_inner, bi = b % p.batch_inner;
+    const float *A = (const float *)p.A + bo * p.sA_out + bi * p.sA_in;
+    const float *B = (const float *)p.B + bo * p.sB_out + bi * p.sB_in;
+    const float *B2 = DUAL ? (const float *)p.B2 + bo * p.sB_out + bi * p.sB_in : nullptr;
+    const int64_t coff = bo * p.sC_out + bi * p.sC_in;
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * (DUAL ? BN / 2 : BN);
+
+    if (p.causal != CAUSAL_NONE && n0 > m0 + BM - 1 + p.causal_offset) {
+        // Entire tile is above the diagonal: no products needed.
+        if (p.causal == CAUSAL_WRITE) {
+            for (int e = threadIdx.x; e < BM * BN; e += THREADS * KG) {
+                const int64_t row = m0 + e / BN, col = n0 + e % BN;
+                if (row < p.M && col < p.N) store_out(p.C, coff + row * p.ldc + col, -INFINITY, p.out_bf16);
+            }
+        }
+        return;
+    }
+
+    int64_t kb = split * p.k_per_split;
+    int64_t ke = min(p.K, kb + p.k_per_split);
+    if (p.kmode == KMODE_LOWER) ke = min(ke, m0 + BM);
+    if (p.kmode == KMODE_UPPER) kb = max(kb, (m0 / BK) * BK);
+    const int ntiles = ke > kb ? (int)((ke - kb + BK - 1) / BK) : 0;
+
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = zero;
+
+    // Register staging sets: PF of them, so that a k-tile's loads go out PF tiles before its split.
+    // The 64 x 64 tile has room for two, which a block alone on its CU needs (measured [4096, 256,
+    // 16384]: 544 -> 302 us unsplit).
+    constexpr int PF = S::WIDE || KG > 1 ? 1 : 2;
+    OA oa[PF];
+    OBL ob[PF];
+    std::conditional_t<DUAL, OBL, char> ob2[PF];
+    TileLoad<OA> ra;
+    TileLoad<OBL> rb, rb2;
+    ra.init(A, p.lda, p.M, p.K, m0, tid);
+    rb.init(B, p.ldb, p.N, p.K, n0, tid);
+    if constexpr (DUAL) rb2.init(B2, p.ldb, p.N, p.K, n0, tid);
+    auto gload = [&](int set, int64_t k0) {
+#pragma unroll
+        for (int q = 0; q < PF; ++q)
+            if (q == set) {
+                ra.load(oa[q], k0, tid);
+                rb.load(ob[q], k0, tid);
+                if constexpr (DUAL) rb2.load(ob2[q], k0, tid);
+            }
+    };
+    // Part `part` of `parts` of a register set's split and LDS writes; k0: its k-tile. A k-contiguous
+    // A's elements past K (the next row's) are zeroed; B's then meet zeros, as an mn-contiguous A's
+    // zeros meet them (a B element past K that is not finite costs the wave its second computation).
+    auto gstore = [&](int set, int64_t k0, int part, int parts) {
+#pragma unroll
+        for (int q = 0; q < PF; ++q)
+            if (q == set) {
+                if constexpr (!TA)
+                    if (part == 0 && k0 + BK > ke) oa[q].mask(ke - k0, tid);
+                oa[q].store(smem, tid, part, parts);
+                ob[q].store(smem + SA, tid, part, parts);
+                if constexpr (DUAL) ob2[q].store(smem + SA + OBL::STAGE_BYTES, tid, part, parts);
+            }
+    };
+    // XPOSE: B as the MFMA's row operand, the block comes out transposed.
+    auto mul = [&](f32x4 &c, const u32x4 &a, const u32x4 &bb) {
+        const bf16x8 av = __builtin_bit_cast(bf16x8, a), bv = __builtin_bit_cast(bf16x8, bb);
+        c = XPOSE ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv, av, c, 0, 0, 0)
+                  : __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, c, 0, 0, 0);
+    };
+
+    if (ntiles > 0) {
+        // One LDS stage, two barriers per k-tile: a wave takes all its fragments of tile t into
+        // registers, and once every wave has, tile t+1 is split and written over it between the
+        // MFMAs of tile t, and the loads of tile t+1+PF go out. The last tile is read again at the
+        // end, into a stage nobody reads.
+        //
+        // The matrix unit rounds its sum once per 8 products, and not evenly: sums drift down by
+        // about 1e-8 of their size per 1000 roundings. So only the leading term product goes into
+        // the running sums; the five small ones, 2^-8 of it and less, have sums of their own
+        // (LOWSUM: for the whole k range; otherwise for one k-tile and strip of 16 rows at a time,
+        // which takes fewer registers). Measured against 64 bits, N(0, 1) data: K = 256 9.0e-8, K =
+        // 4096 2.2e-7 (the FP32 units, summing in k order: 2.9e-7 and 1.1e-6; all six products in
+        // one sum: 2.3e-7 and 5.0e-7, with that drift).
+        constexpr int QA[5] = {2, 0, 1, 1, 0}, QB[5] = {0, 2, 1, 0, 1};
+        constexpr bool LOWSUM = !S::WIDE;
+        f32x4 low[LOWSUM ? FM : 1][FN];
+#pragma unroll
+        for (int i = 0; i < (LOWSUM ? FM : 1); ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) low[i][j] = zero;
+        const int last = ntiles - 1, nt = (ntiles + KG - 1) / KG;
+        auto kt = [&](int t) { return kb + (int64_t)min(t * KG + kg, last) * BK; };
+        u32x4 fa[3][FM], fb[3][FN];
+        auto ktile = [&](int t, int set) {
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+#pragma unroll
+                for (int i = 0; i < FM; ++i) fa[q][i] = OA::frag(smem, wm * WTM + i * 16, q, lane);
+#pragma unroll
+                for (int j = 0; j < FN; ++j) {
+                    if constexpr (DUAL)
+                        fb[q][j] = OBL::frag(smem + SA + wn * OBL::STAGE_BYTES, j * 16, q, lane);
+                    else
+                        fb[q][j] = OB::frag(smem + SA, wn * WTN + j * 16, q, lane);
+                }
+            }
+            __syncthreads();
+            const bool live = KG == 1 || t * KG + kg < ntiles;
+            // Per 16-row strip of the wave's tile: a share of tile t+1's split and LDS writes, then
+            // the strip's products.
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                f32x4 (&lo)[FN] = low[LOWSUM ? i : 0];
+                gstore(set, kt(t + 1), i, FM);
+                if (i == FM - 1) gload(set, kt(t + 1 + PF));
+                if (KG > 1 && !live) continue;
+                if constexpr (!LOWSUM) {
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) lo[j] = zero;
+                }
+#pragma unroll
+                for (int q = 0; q < 5; ++q)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) mul(lo[j], fa[QA[q]][i], fb[QB[q]][j]);
+#pragma unroll
+                for (int j = 0; j < FN; ++j) mul(acc[i][j], fa[0][i], fb[0][j]);
+                if constexpr (!LOWSUM) {
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) acc[i][j] += lo[j];
+                }
+                // Strips in order: left alone, the scheduler gathers all splits first and spills.
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+#pragma unroll
+        for (int q = 0; q < PF; ++q) gload(q, kt(q));
+        gstore(0, kt(0), 0, 1);
+        gload(0, kt(PF));
+        // Tile t+1's registers are set (t + 1) % PF: whole groups of PF tiles in a branch-free body,
+        // then the remaining tiles.
+        int t = 0;
+        for (; t + PF <= nt; t += PF) {
+#pragma unroll
+            for (int q = 0; q < PF; ++q) ktile(t + q, (q + 1) % PF);
+        }
+#pragma unroll
+        for (int q = 0; q + 1 < PF; ++q)
+            if (t + q < nt) ktile(t + q, (q + 1) % PF);
+        if constexpr (LOWSUM) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) acc[i][j] += low[i][j];
+        }
+    }
+    if constexpr (KG > 1) {
+        // The other groups hand their sums over through LDS and are done.
+        constexpr int REGION = THREADS * FM * FN * 16;
+        static_assert((KG - 1) * REGION <= KG * S::SMEM, "the groups' sums fit in the stages");
+        __syncthreads();
+        if (kg > 0) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    *(f32x4 *)(smem0 + (kg - 1) * REGION + ((i * FN + j) * THREADS + tid) * 16) = acc[i][j];
+        }
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int g = 0; g < KG - 1; ++g)
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    acc[i][j] += *(const f32x4 *)(smem0 + g * REGION + ((i * FN + j) * THREADS + tid) * 16);
+    }
+
+    // An element that is not finite (acc * 0 is NaN) may owe that to the split: this wave then takes
+    // its products again on the FP32 units, straight from memory.
+    // Lane l of a 16x16 block holds rows (XPOSE: columns) 4 (l / 16) + r, r = 0..3, and column (row)
+    // l % 16.
+    float nf = 0.f;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                // (columns past M or N may hold anything)
+                const int mn = (lane >> 4) * 4 + r;
+                const int64_t row = m0 + wm * WTM + i * 16 + (XPOSE ? (lane & 15) : mn);
+                const int64_t col = (DUAL ? n0 : n0 + wn * WTN) + j * 16 + (XPOSE ? mn : (lane & 15));
+                nf = row < p.M && col < p.N ? fmaf(acc[i][j][r], 0.f, nf) : nf;
+            }
+    if (__any(nf != nf)) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = zero;
+        const float *Bw = B;
+        int64_t c0 = n0 + wn * WTN;
+        if constexpr (DUAL) {
+            static_assert(WTN == BN / 2, "a wave's columns are all gate or all up");
+            Bw = wn ? B2 : B;
+            c0 = n0;
+        }
+#pragma unroll 1
+        for (int64_t k0 = kb; k0 < ke; k0 += 4) {
+            const int64_t k = k0 + (lane >> 4);
+            float av[FM], bv[FN];
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                const int64_t row = m0 + wm * WTM + i * 16 + (lane & 15);
+                av[i] = 0.f;
+                if (k < ke && row < p.M) av[i] = A[TA ? k * p.lda + row : row * p.lda + k];
+            }
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const int64_t col = c0 + j * 16 + (lane & 15);
+                bv[j] = k < ke && col < p.N ? Bw[TB ? col * p.ldb + k : k * p.ldb + col] : 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    acc[i][j] = XPOSE ? __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j], av[i], acc[i][j], 0, 0, 0)
+                                      : __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+        }
+    }
+
+    if constexpr (XPOSE) {
+        // Lane l of block (i, j) has output row i*16 + l%16 and its consecutive columns j*16 +
+        // 4*(l/16) .. +3.
+        auto each = [&](auto &&f) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    f(acc[i][j], wm * WTM + i * 16 + (lane & 15), wn * WTN + j * 16 + (lane >> 4) * 4);
+        };
+        if constexpr (FIX) {
+            if (p.splits > 1) {
+                // Partial tile of split z at device scope (written through this XCD's L2), then the
+                // arrival count: the tile's last block reads every split's partial at device scope
+                // (missing its own L2), adds them in split order from zero, as the separate
+                // reduction does, and finishes the tile. Offsets are 32-bit (splits * M * N * 4 <
+                // 2^31, checked by the host).
+                const __amdgpu_buffer_rsrc_t prt = __builtin_amdgcn_make_buffer_rsrc(
+                    p.partial, (short)0, (int)(p.splits * p.M * p.N * 4), 0x00020000);
+                each([&](const f32x4 &v, int rl, int cl) __attribute__((always_inline)) {
+                    const int64_t row = m0 + rl, col = n0 + cl;
+                    if (row < p.M && col < p.N)
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), prt,
+                                                               (uint32_t)(((z * p.M + row) * p.N + col) * 4), 0,
+                                                               CP_DEVICE_SCOPE);
+                });
+                __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's partials reached device scope
+                __syncthreads();
+                __shared__ int last_in;
+                if (tid == 0) {
+                    const int old = __hip_atomic_fetch_add(arrive, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    last_in = old == p.splits - 1;
+                    if (last_in) __hip_atomic_store(arrive, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                __syncthreads();
+                if (!last_in) return;
+                each([&](const f32x4 &v, int rl, int cl) __attribute__((always_inline)) {
+                    const int64_t row = m0 + rl, col = n0 + cl;
+                    if (row >= p.M || col >= p.N) return;
+                    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+                    for (int sp = 0; sp < p.splits; ++sp)
+                        sum += sp == z ? v
+                                       : __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                       prt, (uint32_t)(((sp * p.M + row) * p.N + col) * 4),
+                                                                       0, CP_DEVICE_SCOPE));
+                    finish4<true, true>(p, sum, row, col, coff, 0);
+                });
+                return;
+            }
+        }
+        each([&](const f32x4 &v, int rl, int cl) __attribute__((always_inline)) {
+            finish4<true>(p, v, m0 + rl, n0 + cl, coff, z);
+        });
+    } else {
+        // Epilogue through LDS: each wave stages half of its columns at a time with static register
+        // indices, then finishes them row-major with 4-column vectors (DUAL: the gate and up waves of
+        // a row half finish their slice together).
+        constexpr int EC = WTN / 2, EP = EC * 4 + 16, SLAB = WTM * EP;
+        static_assert(KG == 1 && WM * WN * SLAB <= S::SMEM, "epilogue staging fits in the stage");
+        __syncthreads();
+        char *wl = smem + wave * SLAB;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int jj = 0; jj < FN / 2; ++jj)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        *(float *)(wl + (i * 16 + (lane >> 4) * 4 + r) * EP + (jj * 16 + (lane & 15)) * 4) =
+                            acc[i][h * (FN / 2) + jj][r];
+            __syncthreads();
+            if constexpr (DUAL) {
+                static_assert(WN == 2, "one gate and one up wave per row half");
+                const char *gl = smem + (wm * 2) * SLAB, *ul = gl + SLAB;
+                const int pt = wn * 64 + lane;
+                for (int it = 0; it < (WTM * EC + 511) / 512; ++it) {
+                    const int e = (it * 128 + pt) * 4;
+                    if (WTM * EC % 512 != 0 && e >= WTM * EC) break;
+                    const int rl = e / EC, cl = e % EC;
+                    finish_swiglu4<true>(p, *(const f32x4 *)(gl + rl * EP + cl * 4),
+                                                     *(const f32x4 *)(ul + rl * EP + cl * 4), m0 + wm * WTM + rl,
+                                                     n0 + h * EC + cl, coff);
+                }
+            } else {
+                for (int it = 0; it < WTM * EC / 256; ++it) {
+                    const int e = (it * 64 + lane) * 4;
+                    const int rl = e / EC, cl = e % EC;
+                    const f32x4 v = *(const f32x4 *)(wl + rl * EP + cl * 4);
+                    finish4<true>(p, v, m0 + wm * WTM + rl, n0 + wn * WTN + h * EC + cl, coff, z);
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
+template <class S, bool TA, bool TB, bool DUAL>
+__global__ __launch_bounds__(S::THREADS * S::KG, S::WAVES) void gemm_f32_terms(const GemmArgs p) {
+    __shared__ __attribute__((aligned(16))) char smem[S::KG * S::SMEM];
+    gemm_f32_block<S, TA, TB, DUAL>(p, blockIdx.x, blockIdx.y, smem);
+}
+
+// A group of GEMMs: 64 x 64 tiles, batch 1, one split count for the group. Split-K partial sums go to
+// each problem's own region, and each tile's last block to arrive adds its splits and finishes it.
+template <bool TA, bool TB>
+__global__ __launch_bounds__(S64::THREADS, S64::WAVES) void gemm_f32_terms_group(const GemmGroupArgs grp) {
+    __shared__ __attribute__((aligned(16))) char smem[S64::SMEM];
+    int gi, split, tile;
+    if (!group_block(grp, gi, split, tile)) return;
+    const GemmArgs p = grp.g[gi];  // a copy: through the reference the whole argument went to scratch
+    gemm_f32_block<S64, TA, TB, false, true>(p, tile, split, smem, grp.arrive + grp.cstart[gi] + tile);
+}
+
+template <class S, bool TA, bool TB, bool DUAL>
+void go(const GemmArgs &a, dim3 grid, hipStream_t s) {
+    hipLaunchKernelGGL((gemm_f32_terms<S, TA, TB, DUAL>), grid, dim3(S::THREADS * S::KG), 0, s, a);
+}
+
+// bm x bn: the output tile (SwiGLU: half as wide as its B tile).
+template <bool TA, bool TB>
+void launch_plain(int bm, int bn, const GemmArgs &a, dim3 grid, hipStream_t s) {
+    if constexpr (!TA)
+        if (bm == 256) return go<S256, TA, TB, false>(a, grid, s);
+    if (bm == 128) return go<S128, TA, TB, false>(a, grid, s);
+    if (bn == 32) return go<S6432, TA, TB, false>(a, grid, s);
+    go<S64, TA, TB, false>(a, grid, s);
+}
+
+// The tiles as the planner prices them, in microseconds: a k-tile of a block that shares its CU (its
+// share of the CU's time) and of one that has it alone, and a round's prologue and epilogue, fitted on
+// timings of every tile and split on the TINY step's shapes, ragged ones and 4096^3.
+struct Tile {
+    int bm, bn, occ;  // occ: blocks a CU runs at once
+    double shared, alone, round;
+};
+// 256 x 128 before 128 x 128, which it beats by 3% where both fill the GPU (4096^3 651 against 674 us,
+// [4096, 256, 16384] 197 against 203).
+constexpr Tile T256{256, 128, 1, 2.55, 2.55, 8.0}, T128{128, 128, 2, 1.31, 1.75, 4.5},
+    T64{64, 64, 3, 0.45, 0.60, 3.0}, T6432{64, 32, 2, 0.268, 0.30, 3.0};
+
+struct Plan {
+    int bm, bn, splits;
+    int64_t k_per_split;
+};
+
+// One launch of `blocks` blocks of ksteps k-tiles, in seconds.
+double launch_time(const Tile &t, int64_t blocks, int64_t ksteps, int64_t cus) {
+    const int64_t per_cu = cdiv(blocks, cus), conc = std::min<int64_t>(per_cu, t.occ);
+    return 1e-6 * cdiv(per_cu, t.occ) * (t.round + ksteps * std::max(conc * t.shared, t.alone));
+}
+
+// Picks the tile and a power-of-two split count, lowest price first. Near ties (3%) keep the earlier
+// plan, except that between two unsplit plans the one with more blocks wins (more loads in flight per
+// k-step); the 64 x 32 tile has to win outright.
+Plan choose_plan(const GemmArgs &a, int64_t cus, bool ta, double *est) {
+    constexpr int bk = ET<float>::BK;
+    const bool plain = !a.dual && a.causal == CAUSAL_NONE && a.kmode == KMODE_FULL;
+    const int64_t kall = std::max<int64_t>(1, cdiv(a.K, bk)) * bk;
+    Plan best{64, a.dual ? 32 : 64, 1, kall};
+    double best_t = 1e30;
+    int64_t best_blocks = 0;
+    for (const Tile &tile : {T256, T128, T64, T6432}) {
+        if (tile.bm != tile.bn && !plain) continue;
+        if (tile.bm == 256 && (ta || a.swiglu_bwd || a.rope_table)) continue;
+        const int bn = a.dual ? tile.bn / 2 : tile.bn;
+        const int64_t tiles = cdiv(a.M, tile.bm) * cdiv(a.N, bn) * a.batch;
+        for (int s = 1; s <= 32; s *= 2) {
+            if (s > 1 && (!plain || a.no_split)) break;
+            const int64_t kps = s == 1 ? kall : cdiv(cdiv(a.K, s), bk) * bk;
+            if (s > 1 && kps < 4 * bk) break;
+            const int64_t splits = s > 1 ? cdiv(a.K, kps) : 1, blocks = tiles * splits;
+            double t = launch_time(tile, blocks, kps / bk, cus);
+            if (splits > 1) t += 2.0 * splits * a.M * a.N * a.batch * 4.0 / 4e12 + 4e-6;  // partial sums, reduction
+            const bool better = t < best_t * 0.97;
+            const bool tie_more_blocks = t < best_t * 1.03 && splits == 1 && best.splits == 1 &&
+                                         blocks > best_blocks && tile.bn != 32;
+            if (better || tie_more_blocks) {
+                best_t = better ? t : std::min(t, best_t);
+                best = Plan{tile.bm, bn, (int)splits, kps};
+                best_blocks = blocks;
+            }
+        }
+    }
+    if (est) *est = best_t;
+    return best;
+}
+
+int64_t cus_of(const it_context *ctx) { return ctx->num_cus > 0 ? ctx->num_cus : 256; }
+
+// 4-column vectors of an FP32 output need an element's alignment only.
+void any_alignment(GemmArgs &a) { a.c_vec_ok = a.c_vec_ok || !a.out_bf16; }
+
+}  // namespace
+
+bool f32_terms_applicable(const GemmArgs &a, bool ta, bool tb) {
+    // A few rows wait on latency, not on the matrix units: M = 1, N = 768, K = 256 takes 6.7 us here
+    // and 6.0 on the FP32 units' 64 x 32 tile, which loads two k-tiles ahead.
+    return a.M > 16 && !a.f32_units && !a.a_kscale && !a.xent_stats && spans_fit(a, ta, tb);
+}
+
+it_status launch_gemm_f32(it_context *ctx, bool ta, bool tb, GemmArgs a, const char *tag) {
+    Plan plan = choose_plan(a, cus_of(ctx), ta, nullptr);
+#ifdef IT_TUNING
+    // Planner sweeps only (a tuning build): IT_PLAN="tile,splits[,width]" forces the plan.
+    if (const char *env = std::getenv("IT_PLAN")) {
+        int bm = 0, sp = 0, bn = 0;
+        const int n = std::sscanf(env, "%d,%d,%d", &bm, &sp, &bn);
+        if (n >= 2) plan = Plan{bm, a.dual ? bm / 2 : n == 3 ? bn : bm, sp, cdiv(cdiv(a.K, sp), 32) * 32};
+    }
+#endif
+    a.tiles_m = (int)cdiv(a.M, plan.bm);
+    a.tiles_n = (int)cdiv(a.N, plan.bn);
+    a.k_per_split = plan.k_per_split;
+    a.splits = (int)std::max<int64_t>(1, cdiv(a.K, plan.k_per_split));
+    any_alignment(a);
+    if (a.splits > 1) {
+        void *ws = nullptr;
+        const it_status st = ensure_scratch(ctx, (size_t)a.splits * a.batch * a.M * a.N * sizeof(float), &ws);
+        if (st != IT_OK) return st;
+        a.partial = (float *)ws;
+    }
+    const int64_t gx = (int64_t)a.tiles_m * a.tiles_n, gy = a.batch * a.splits;
+    if (gx > 0x7fffffff || gy > 65535)
+        return fail(IT_ERR_DIMS, "it_gemm: grid too large (tiles " + std::to_string(gx) + ", batch*splits " +
+                                     std::to_string(gy) + ")");
+    const dim3 grid((unsigned)gx, (unsigned)gy);
+    std::string key;
+    hipEvent_t ev = nullptr;
+    if (ctx->profiling) {
+        char buf[192];
+        std::snprintf(buf, sizeof(buf), "gemm_f32_%c%c_%dx%d%s%s|%s[%lld,%lld,%lld]x%lld s%d", ta ? 'T' : 'N',
+                      tb ? 'T' : 'N', plan.bm, a.dual ? plan.bm : plan.bn, a.dual ? "_swiglu" : "",
+                      a.causal || a.kmode ? "_causal" : "", tag ? tag : "", (long long)a.M, (long long)a.N,
+                      (long long)a.K, (long long)a.batch, a.splits);
+        key = buf;
+        profile_begin(ctx, key, &ev);
+    }
+    hipStream_t s = ctx->stream;
+    if (a.dual) {  // X.W^T (checked by the caller)
+        if (plan.bm == 128) go<S128, false, true, true>(a, grid, s);
+        else go<S64, false, true, true>(a, grid, s);
+    } else if (!ta && !tb) {
+        launch_plain<false, false>(plan.bm, plan.bn, a, grid, s);
+    } else if (!ta && tb) {
+        launch_plain<false, true>(plan.bm, plan.bn, a, grid, s);
+    } else if (ta && !tb) {
+        launch_plain<true, false>(plan.bm, plan.bn, a, grid, s);
+    } else {
+        launch_plain<true, true>(plan.bm, plan.bn, a, grid, s);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail_hip(e, "gemm_f32_terms launch");
+    if (a.splits > 1) {
+        const it_status st = launch_splitk_reduce(s, a);
+        if (st != IT_OK) return st;
+    }
+    if (ctx->profiling) profile_end(ctx, key, ev);
+    return IT_OK;
+}
+
+// One gemm_f32_terms_group launch (64 x 64 tiles, one split count for the group; each tile's last split
+// block adds the partial sums) where the planner prices it below the separate plans.
+bool launch_gemm_f32_group(it_context *ctx, bool ta, bool tb, const GemmArgs *args, int count, const char *tag,
+                           it_status *status) {
+    constexpr int bk = ET<float>::BK;
+    const int64_t cus = cus_of(ctx);
+    if (count < 2) return false;
+    double separate = 0.0;
+    for (int i = 0; i < count; ++i) {
+        const GemmArgs &a = args[i];
+        if (a.batch != 1 || a.dual || a.causal != CAUSAL_NONE || a.kmode != KMODE_FULL || a.swiglu_bwd || a.K <= 0 ||
+            a.N % 4 != 0 || a.no_split)
+            return false;
+        double t = 0.0;
+        choose_plan(a, cus, ta, &t);
+        separate += t;
+    }
+    // The model of the group at one split count s. The XCD schedule takes at most count * s + 7
+    // chunks (a chunk per GEMM and split, plus one more where an XCD's share ends inside one), so s
+    // stays where that fits the table.
+    double best_t = 1e30;
+    int best_s = 0;
+    for (int s = 1; s <= 32 && count * s + 7 <= GROUP_CHUNKS; ++s) {
+        int64_t blocks = 0, ksteps = 0;
+        double traffic = 0.0;
+        bool ok = true;
+        for (int i = 0; i < count && ok; ++i) {
+            const GemmArgs &a = args[i];
+            const int64_t kps = cdiv(cdiv(a.K, s), bk) * bk;
+            ok = s == 1 || kps >= 4 * bk;
+            const int64_t splits = s > 1 ? cdiv(a.K, kps) : 1;
+            blocks += cdiv(a.M, 64) * cdiv(a.N, 64) * splits;
+            ksteps = std::max(ksteps, cdiv(kps, bk));
+            if (splits > 1) traffic += 2.0 * splits * a.M * a.N * 4.0;
+        }
+        if (!ok) break;
+        double t = launch_time(T64, blocks, ksteps, cus);
+        if (traffic > 0.0) t += traffic / 4e12 + 4e-6;  // partial sums out and back, the tiles' last-block sums
+        if (t < best_t) {
+            best_t = t;
+            best_s = s;
+        }
+    }
+#ifdef IT_TUNING
+    // Planner sweeps only (a tuning build): IT_GROUP_SPLITS forces the group's split count.
+    if (const char *env = std::getenv("IT_GROUP_SPLITS")) {
+        best_s = std::max(1, std::min(32, std::atoi(env)));
+        best_t = 0.0;
+    }
+#endif
+    if (!best_s || best_t >= 0.97 * separate) return false;
+    GemmGroupArgs grp{};
+    grp.count = count;
+    int64_t scratch = 0, tiles = 0;
+    bool split_any = false;
+    for (int i = 0; i < count; ++i) {
+        GemmArgs &a = grp.g[i];
+        a = args[i];
+        const int64_t kps = cdiv(cdiv(a.K, best_s), bk) * bk;
+        a.splits = best_s > 1 ? (int)cdiv(a.K, kps) : 1;
+        a.k_per_split = best_s > 1 ? kps : cdiv(a.K, bk) * bk;
+        a.tiles_m = (int)cdiv(a.M, 64);
+        a.tiles_n = (int)cdiv(a.N, 64);
+        any_alignment(a);
+        grp.cstart[i] = (int)tiles;
+        tiles += (int64_t)a.tiles_m * a.tiles_n;
+        if (a.splits > 1) {
+            // the in-kernel sum addresses a problem's partials with 32-bit byte offsets
+            if ((int64_t)a.splits * a.M * a.N * 4 >= (1ll << 31)) return false;
+            split_any = true;
+            scratch += (int64_t)a.splits * a.M * a.N;
+        }
+    }
+    if (tiles > COUNTERS) return false;
+    grp.cstart[count] = (int)tiles;
+    const int grid_blocks = xcd_schedule(grp);
+    if (!grid_blocks) return false;
+    if (split_any) {
+        *status = ensure_counters(ctx, &grp.arrive);
+        if (*status != IT_OK) return true;
+        void *ws = nullptr;
+        *status = ensure_scratch(ctx, (size_t)scratch * sizeof(float), &ws);
+        if (*status != IT_OK) return true;
+        float *part = (float *)ws;
+        for (int i = 0; i < count; ++i)
+            if (grp.g[i].splits > 1) {
+                grp.g[i].partial = part;
+                part += (int64_t)grp.g[i].splits * grp.g[i].M * grp.g[i].N;
+            }
+    }
+    std::string key;
+    hipEvent_t ev = nullptr;
+    if (ctx->profiling) {
+        key = std::string("gemm_f32_") + (ta ? 'T' : 'N') + (tb ? 'T' : 'N') + "_64x64_group|" + (tag ? tag : "");
+        for (int i = 0; i < count; ++i)
+            key += (i ? "+[" : "[") + std::to_string(args[i].M) + "," + std::to_string(args[i].N) + "," +
+                   std::to_string(args[i].K) + "]";
+        key += "x1 s" + std::to_string(best_s);
+        profile_begin(ctx, key, &ev);
+    }
+    const dim3 grid((unsigned)grid_blocks), block(S64::THREADS);
+    if (!ta && tb) hipLaunchKernelGGL((gemm_f32_terms_group<false, true>), grid, block, 0, ctx->stream, grp);
+    else if (!ta && !tb) hipLaunchKernelGGL((gemm_f32_terms_group<false, false>), grid, block, 0, ctx->stream, grp);
+    else if (ta && !tb) hipLaunchKernelGGL((gemm_f32_terms_group<true, false>), grid, block, 0, ctx->stream, grp);
+    else hipLaunchKernelGGL((gemm_f32_terms_group<true, true>), grid, block, 0, ctx->stream, grp);
+    const hipError_t e = hipGetLastError();
+    *status = e == hipSuccess ? IT_OK : fail_hip(e, "gemm group launch");
+    if (ctx->profiling && *status == IT_OK) profile_end(ctx, key, ev);
+    return true;
+}
+
+}  // namespace it

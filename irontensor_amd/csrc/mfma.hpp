@@ -28,6 +28,26 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 
+// Two FP32 values as three BF16 terms each, x = t0 + t1 + t2 (packed in pairs, the first value low):
+// every term is the round-to-nearest-even of what the terms before it leave, and those differences
+// are exact, so the terms carry 3 x 8 = 24 significand bits (down to BF16's smallest step, 2^-133:
+// values below 2^-110 lose bits under it). An infinity, a NaN or a value that rounds up to 2^128
+// gives a NaN term.
+struct Bf16x3 {
+    uint32_t t[3];
+};
+__device__ __forceinline__ Bf16x3 split_bf16x3(uint32_t bits0, uint32_t bits1) {
+    float a = __uint_as_float(bits0), b = __uint_as_float(bits1);
+    Bf16x3 r;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        r.t[p] = pack_bf16x2(a, b);
+        a -= __uint_as_float(r.t[p] << 16);
+        b -= __uint_as_float(r.t[p] & 0xffff0000u);
+    }
+    return r;
+}
+
 __device__ __forceinline__ uint16_t f32_to_bf16_rne(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }

@@ -27,6 +27,10 @@ attention kernels), and the row/elementwise ops of kernels_train.hip. The MI355X
     forked once per layer (dw_fork="layer": each fork costs several microseconds of idle GPU
     inside the graph, so that beat one fork per GEMM, "gemm", 2.80 against 2.85 ms per TINY step
     before the grouping);
+  * the products sum on the FP32 units (IT_EPI_F32_UNITS) by default: Lion steps by the sign of its
+    update, so a run's weights follow the rounding of its gradients, and these sums keep a run bit
+    for bit what it was. f32_units=False takes the library's default FP32 products (BF16 terms:
+    nearer to the exact sums, a 10% faster TINY step, other roundings);
   * the gradient norm, the clip factor and the learning rate stay on the device (Lion reads them
     from memory), so a step has no host synchronisation and captures into one HIP graph.
 
@@ -57,7 +61,8 @@ class TrainStep:
                  lr: float = 3e-4, beta1: float = 0.9, beta2: float = 0.99, weight_decay: float = 0.1,
                  max_grad_norm: float = 1.0, eps: float = 1e-5, rope_base: float = 10000.0,
                  overlap_weight_grads: bool = False, fused_attention: Optional[bool] = None,
-                 xent_operand: bool = False, dw_fork: str = "layer", group_weight_grads: bool = True):
+                 xent_operand: bool = False, dw_fork: str = "layer", group_weight_grads: bool = True,
+                 f32_units: bool = True):
         s = shape
         if s.heads * s.head_dim != s.hidden:
             raise ValueError("heads * head_dim must equal hidden")
@@ -71,6 +76,7 @@ class TrainStep:
         self.overlap = overlap_weight_grads
         self.group_weight_grads = bool(group_weight_grads)
         self.fused = (s.head_dim == 64) if fused_attention is None else bool(fused_attention)
+        self.f32_units = bool(f32_units)
         self.xent_operand = bool(xent_operand)
         if dw_fork not in ("gemm", "layer"):
             raise ValueError("dw_fork is 'gemm' or 'layer'")
@@ -190,15 +196,23 @@ class TrainStep:
         check(self.lib.it_memcpy_h2d(self.h, C.c_void_p(self.lr_dev.ptr), v.ctypes.data_as(C.c_void_p), 4), "lr")
 
     # ---------------------------------------------------------------- launch helpers
-    @staticmethod
-    def _call(A: Tensor, B: Tensor, Cout: Tensor, ta: bool, tb: bool, M, N, K,
+    def _epi(self, epi: Optional[_lib.Epilogue]) -> Optional[_lib.Epilogue]:
+        """The call's epilogue, asking for the FP32 units when the step does."""
+        if self.f32_units:
+            epi = epi if epi is not None else _lib.Epilogue()
+            epi.flags |= _lib.IT_EPI_F32_UNITS
+        return epi
+
+    def _call(self, A: Tensor, B: Tensor, Cout: Tensor, ta: bool, tb: bool, M, N, K,
               epi: Optional[_lib.Epilogue] = None) -> _lib.GemmCall:
         """it_gemm's arguments for one FP32 GEMM of the step (batch 1, alpha 1, beta 0)."""
+        epi = self._epi(epi)
         return _lib.GemmCall(int(ta), int(tb), M, N, K, 1.0, A.ptr, A.shape()[-1], 0, B.ptr, B.shape()[-1], 0,
                              0.0, Cout.ptr, Cout.shape()[-1], 0, 1, C.pointer(epi) if epi is not None else None)
 
     def _gemm(self, name, A: Tensor, B: Tensor, Cout: Tensor, ta: bool, tb: bool, M, N, K,
               epi: Optional[_lib.Epilogue] = None):
+        epi = self._epi(epi)
         st = self.lib.it_gemm(self.h, 0, 0, int(ta), int(tb), M, N, K, 1.0, C.c_void_p(A.ptr), A.shape()[-1], 0,
                               C.c_void_p(B.ptr), B.shape()[-1], 0, 0.0, C.c_void_p(Cout.ptr), Cout.shape()[-1], 0, 1,
                               C.byref(epi) if epi is not None else None)

@@ -1,0 +1,133 @@
+"""FP32 products as BF16 terms (the default it_gemm FP32 path) at the edges of their tiles and on
+operands the split has to hand over to the FP32 units.
+
+Bound per element, against the float64 product of the same operands: an element split into three
+BF16 terms keeps 24 significand bits, the left-out term products are below 2^-24 of a product, and
+the running sums round once per 8 products, so |error| <= (K / 8 + 16) 2^-23 (|A|.|B|)_ij.
+"""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from irontensor_amd import _lib, synth
+from tests.numerics import op
+
+pytestmark = pytest.mark.gpu
+
+LAYOUTS = [(0, 0), (0, 1), (1, 0), (1, 1)]
+
+
+def _operands(seed, m, n, k, ta, tb):
+    a = synth.normal(seed, (k, m) if ta else (m, k))
+    b = synth.normal(seed + 1, (n, k) if tb else (k, n), std=0.02)
+    return a, b
+
+
+def _check(got, a, b, ta, tb, k, extra=0.0):
+    A, B = op(a, ta).astype(np.float64), op(b, tb).astype(np.float64)
+    bound = (k / 8 + 16) * 2.0 ** -23 * (np.abs(A) @ np.abs(B)) + 1e-30
+    worst = float(np.max(np.abs(got - (A @ B + extra)) / bound))
+    assert worst <= 1.0, f"error {worst:.2f} times its bound"
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 768, 256), (63, 65, 31), (64, 32, 33), (65, 33, 32), (129, 127, 97),
+                                   (300, 701, 1000), (128, 128, 64), (1025, 515, 70), (257, 40, 3000)])
+def test_layouts_and_edges(it, m, n, k, ta, tb):
+    a, b = _operands(m + 7 * n + k, m, n, k, ta, tb)
+    c = it.gemm(it.Tensor.from_f32_slice(a, a.shape), it.Tensor.from_f32_slice(b, b.shape), trans_a=bool(ta),
+                trans_b=bool(tb))
+    _check(c.numpy(), a, b, ta, tb, k)
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("tile_n,m,n,k", [(256, 512, 384, 4096), (128, 640, 1152, 96), (64, 192, 200, 40)])
+def test_strided_unaligned_operands(it, tile_n, m, n, k, ta, tb):
+    """Rows at any element alignment: operands and output inside wider buffers, starting at odd columns,
+    whose surrounding elements are NaN (they may be read past K and past an edge, never used) or must
+    stay untouched."""
+    a, b = _operands(31 + m, m, n, k, ta, tb)
+    ctx = it.Context.global_()
+
+    def wide(x, fill):
+        w = np.full((x.shape[0] + 2, x.shape[1] + 7), fill, np.float32)
+        w[1:-1, 3:-4] = x
+        return it.Tensor.from_f32_slice(w, list(w.shape)), w.shape[1]
+
+    (A, lda), (B, ldb) = wide(a, np.nan), wide(b, np.nan)
+    Cw, ldc = wide(np.zeros((m, n), np.float32), 7.0)
+    ptr = lambda t, ld: C.c_void_p(t.ptr + 4 * (ld + 3))
+    st = ctx.lib.it_gemm(ctx.handle, 0, 0, ta, tb, m, n, k, 1.0, ptr(A, lda), lda, 0, ptr(B, ldb), ldb, 0, 0.0,
+                         ptr(Cw, ldc), ldc, 0, 1, None)
+    assert st == 0
+    got = Cw.numpy()
+    _check(got[1:-1, 3:-4], a, b, ta, tb, k)
+    edge = got.copy()
+    edge[1:-1, 3:-4] = 7.0
+    assert np.all(edge == 7.0)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0)])
+@pytest.mark.parametrize("m,n,k", [(70, 66, 80), (300, 260, 520)])
+def test_nonfinite_and_extreme_operands(it, m, n, k, ta, tb):
+    """An infinity, a NaN, the type's largest value and subnormals give what the FP32 units give: the
+    same non-finite elements, and the finite ones within the bound."""
+    a, b = _operands(5, m, n, k, ta, tb)
+    big = np.finfo(np.float32).max
+    va, vb = op(a, ta), op(b, tb)  # views
+    va[3, 5] = np.inf
+    va[17, 2] = -np.inf
+    va[40, k - 1] = np.nan
+    va[50, 7] = big
+    va[51, 7] = -big
+    vb[9, 11] = np.inf
+    va[60, :] = 1e-40
+    A, B = it.Tensor.from_f32_slice(a, a.shape), it.Tensor.from_f32_slice(b, b.shape)
+    got = it.gemm(A, B, trans_a=bool(ta), trans_b=bool(tb)).numpy()
+    units = it.Tensor.empty([m, n])
+    epi = _lib.Epilogue(flags=_lib.IT_EPI_F32_UNITS)
+    st = A.ctx.lib.it_gemm(A.ctx.handle, 0, 0, ta, tb, m, n, k, 1.0, C.c_void_p(A.ptr), a.shape[1], 0,
+                           C.c_void_p(B.ptr), b.shape[1], 0, 0.0, C.c_void_p(units.ptr), n, 0, 1, C.byref(epi))
+    assert st == 0
+    ref = units.numpy()
+    fine = np.isfinite(ref)
+    assert np.array_equal(fine, np.isfinite(got)) and np.array_equal(np.isnan(ref), np.isnan(got))
+    assert np.array_equal(ref[~fine & ~np.isnan(ref)], got[~fine & ~np.isnan(ref)])
+    with np.errstate(all="ignore"):
+        A64, B64 = va.astype(np.float64), vb.astype(np.float64)
+        exact, size = A64 @ B64, np.abs(A64) @ np.abs(B64)
+        err = np.abs(got.astype(np.float64) - exact)[fine]
+        # BF16's smallest step is 2^-133: an element's terms miss it by half of that at most.
+        tiny = 2.0 ** -134 * np.broadcast_to(np.abs(B64).sum(0), exact.shape)[fine] + 2.0 ** -140
+    assert np.all(err <= (k / 8 + 16) * 2.0 ** -23 * size[fine] + tiny)
+
+
+@pytest.mark.parametrize("rows,h,f", [(65, 33, 49), (200, 256, 688), (1024, 128, 2048)])
+def test_swiglu_and_bias(it, rows, h, f):
+    x, wg, wu = synth.normal(1, (rows, h)), synth.normal(2, (f, h), std=0.05), synth.normal(3, (f, h), std=0.05)
+    bias = synth.normal(4, (2 * f,), std=0.1)
+    T = it.Tensor.from_f32_slice
+    hh, g, u = it.swiglu_up(T(x, x.shape), T(wg, wg.shape), T(wu, wu.shape), bias=T(bias, [2 * f]))
+    _check(g.numpy(), x, wg, 0, 1, h, bias[None, :f].astype(np.float64))
+    _check(u.numpy(), x, wu, 0, 1, h, bias[None, f:].astype(np.float64))
+    gate, up = g.numpy().astype(np.float64), u.numpy().astype(np.float64)
+    ref = gate / (1 + np.exp(-gate)) * up
+    assert np.max(np.abs(hh.numpy() - ref)) <= 4e-6 * np.max(np.abs(ref))
+
+
+def test_training_step_on_the_fp32_units_or_terms(it):
+    """f32_units=False takes the terms: the first step's gradients agree to FP32 rounding."""
+    from irontensor_amd.step import ModelShape
+    from irontensor_amd.train import TrainStep
+
+    shape = ModelShape("small", 2, 128, 2, 64, 176, 1000, 2, 64)
+    grads = []
+    for units in (True, False):
+        st = TrainStep(shape, seed=5, f32_units=units)
+        st.step()
+        grads.append([t.numpy().astype(np.float64) for t in st.grads])
+    for x, y in zip(*grads):
+        assert np.linalg.norm(x - y) <= 2e-5 * np.linalg.norm(x)
