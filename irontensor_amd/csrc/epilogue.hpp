@@ -11,8 +11,9 @@
 namespace it {
 namespace {
 
-// Four FP32 values of an output row: 128-bit accesses that need an element's alignment only.
+// Four values of an output row, FP32 and BF16: vector accesses that need an element's alignment only.
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
 
 __device__ __forceinline__ float load_out(const void *C, int64_t idx, int bf16) {
     return bf16 ? bf16_to_f32(((const uint16_t *)C)[idx]) : ((const float *)C)[idx];
@@ -62,8 +63,8 @@ __device__ __forceinline__ void finish4(const GemmArgs &p, f32x4 v, int64_t row,
     const bool full = !EDGE || col + 4 <= p.N;
     if (!FINAL && p.splits > 1) {
         float *dst = p.partial + (z * p.M + row) * p.N + col;
-        if (full && p.N % 4 == 0) {
-            *(f32x4 *)dst = v;
+        if (full) {
+            *(f32x4_any *)dst = v;
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -78,7 +79,7 @@ __device__ __forceinline__ void finish4(const GemmArgs &p, f32x4 v, int64_t row,
             const int64_t gi = row * p.N + col;
             f32x4 g, u, dg, du;
             if (p.out_bf16) {
-                const u32x2 gh = *(const u32x2 *)((const uint16_t *)p.G + gi), uh = *(const u32x2 *)((const uint16_t *)p.U + gi);
+                const u32x2 gh = *(const u32x2_any *)((const uint16_t *)p.G + gi), uh = *(const u32x2_any *)((const uint16_t *)p.U + gi);
                 g = f32x4{__uint_as_float(gh[0] << 16), __uint_as_float(gh[0] & 0xffff0000u),
                           __uint_as_float(gh[1] << 16), __uint_as_float(gh[1] & 0xffff0000u)};
                 u = f32x4{__uint_as_float(uh[0] << 16), __uint_as_float(uh[0] & 0xffff0000u),
@@ -94,8 +95,8 @@ __device__ __forceinline__ void finish4(const GemmArgs &p, f32x4 v, int64_t row,
                 du[e] = b;
             }
             if (p.out_bf16) {
-                *(u32x2 *)((uint16_t *)p.C + idx) = u32x2{pack_bf16x2(dg[0], dg[1]), pack_bf16x2(dg[2], dg[3])};
-                *(u32x2 *)((uint16_t *)p.C + idx + p.N) = u32x2{pack_bf16x2(du[0], du[1]), pack_bf16x2(du[2], du[3])};
+                *(u32x2_any *)((uint16_t *)p.C + idx) = u32x2{pack_bf16x2(dg[0], dg[1]), pack_bf16x2(dg[2], dg[3])};
+                *(u32x2_any *)((uint16_t *)p.C + idx + p.N) = u32x2{pack_bf16x2(du[0], du[1]), pack_bf16x2(du[2], du[3])};
             } else {
                 *(f32x4_any *)((float *)p.C + idx) = dg;
                 *(f32x4_any *)((float *)p.C + idx + p.N) = du;
@@ -106,7 +107,7 @@ __device__ __forceinline__ void finish4(const GemmArgs &p, f32x4 v, int64_t row,
         if (p.beta != 0.f) {
             f32x4 old;
             if (p.out_bf16) {
-                const u32x2 o = *(const u32x2 *)((const uint16_t *)p.C + idx);
+                const u32x2 o = *(const u32x2_any *)((const uint16_t *)p.C + idx);
                 old = f32x4{__uint_as_float(o[0] << 16), __uint_as_float(o[0] & 0xffff0000u),
                             __uint_as_float(o[1] << 16), __uint_as_float(o[1] & 0xffff0000u)};
             } else {
@@ -139,7 +140,7 @@ __device__ __forceinline__ void finish4(const GemmArgs &p, f32x4 v, int64_t row,
             u32x2 o;
             o[0] = pack_bf16x2(v[0], v[1]);
             o[1] = pack_bf16x2(v[2], v[3]);
-            *(u32x2 *)((uint16_t *)p.C + idx) = o;
+            *(u32x2_any *)((uint16_t *)p.C + idx) = o;
         } else {
             *(f32x4_any *)((float *)p.C + idx) = v;
         }
@@ -174,7 +175,7 @@ __device__ __forceinline__ void finish_swiglu4(const GemmArgs &p, f32x4 g, f32x4
     if (full && p.c_vec_ok) {
         if (p.out_bf16) {
             auto st = [&](void *dst, f32x4 v) {
-                *(u32x2 *)((uint16_t *)dst + idx) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+                *(u32x2_any *)((uint16_t *)dst + idx) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
             };
             if (p.G) st(p.G, g);
             if (p.U) st(p.U, u);

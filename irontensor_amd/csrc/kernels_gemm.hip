@@ -829,9 +829,12 @@ void gemm_bf16_256(const GemmArgs p) {
 //     distinct 16-byte bank groups.
 // The 256 x 128 form (FB = 2: each wave 128 x 64) stages 128 B rows: 4 load instructions per wave,
 // an mn-contiguous k-row of 256 bytes (16 chunks, the same XOR, 4 k-rows per load instruction).
-// Whole tiles only (M a multiple of 256, N of the tile width, K of 128); no k limits or masked
-// epilogues.
+// K a multiple of 128 (64 for the 128 x 128 form); rows and columns past M and N are not read, and a
+// tile that passes them (EDGE) finishes with bounds checks. No k limits or causal epilogues.
+// The range check works on whole dwords: an odd number of elements ends with the (4-byte aligned)
+// dword that holds the last one.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t dtl_rsrc(const void *base, int64_t bytes) {
+    bytes = (bytes + 3) & ~int64_t(3);
     const int n = bytes > 0x7fffffff ? 0x7fffffff : (int)bytes;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, n, 0x00020000);
 }
@@ -860,13 +863,15 @@ struct DtlOperand {
     uint32_t voff[NI];
     uint32_t kstride;  // bytes per k of the global operand (2 for k-contiguous, 2 ld otherwise)
 
-    // base: element (row 0, k kb) of this block; krange: k extent of this block's split. A
-    // k-contiguous operand may take the rows from `row_shift` on from a second matrix (the up
-    // weight of the SwiGLU dual form: this wave's rows are then rows r - row_shift of `base`).
-    __device__ __forceinline__ void init(const uint16_t *base, int64_t ld, int64_t krange, int wave, int lane,
-                                         int row_shift = 0) {
+    // base: element (row 0, k kb) of this block, with `rows` rows of the operand from there on and a k
+    // extent of `krange` in this block's split: the descriptor ends with them, so rows past an edge
+    // are not read. A k-contiguous operand may take the rows from `row_shift` on from a second matrix
+    // (the up weight of the SwiGLU dual form: this wave's rows are then rows r - row_shift of `base`).
+    __device__ __forceinline__ void init(const uint16_t *base, int64_t ld, int64_t rows, int64_t krange, int wave,
+                                         int lane, int row_shift = 0) {
+        if (rows > ROWS - row_shift) rows = ROWS - row_shift;
         if constexpr (KCONTIG) {
-            rsrc = dtl_rsrc(base, (int64_t)(ROWS - row_shift) * ld * 2);
+            rsrc = dtl_rsrc(base, ((rows - 1) * ld + krange) * 2);
             kstride = 2;
 #pragma unroll
             for (int j = 0; j < NI; ++j) {
@@ -875,7 +880,7 @@ struct DtlOperand {
                 voff[j] = (uint32_t)(((r - row_shift) * ld + c * 8) * 2);
             }
         } else {
-            rsrc = dtl_rsrc(base, krange * ld * 2);
+            rsrc = dtl_rsrc(base, ((krange - 1) * ld + rows) * 2);
             kstride = (uint32_t)(ld * 2);
 #pragma unroll
             for (int j = 0; j < NI; ++j) {
@@ -928,16 +933,16 @@ struct DtlOperand {
 
 // The k loop of one tile: acc = op(A)[m0.., kb..] . op(B)[.., n0..] over `ntiles` k-tiles (even).
 // A and B point at element (row 0, k kb) of the tile's operands; `krange` bounds an mn-contiguous
-// operand's buffer. The caller synchronises the block before (the stages may still be read) and
-// after (the epilogue reuses them).
+// operand's buffer; with EDGE, rows_a and rows_b bound both operands' rows. The caller synchronises the
+// block before (the stages may still be read) and after (the epilogue reuses them).
 // s_waitcnt immediate: vmcnt(vm) lgkmcnt(lgkm), expcnt not waited on.
 constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8); }
 
-template <bool TA, bool TB, bool DUAL, int FB, bool OPAQUE = (FB == 2), int FA = 4, int NSX = 0>
+template <bool TA, bool TB, bool DUAL, int FB, bool EDGE, bool OPAQUE = (FB == 2), int FA = 4, int NSX = 0>
 __device__ __forceinline__ void dtl_tile(const GemmArgs &p, char *__restrict__ st0, char *__restrict__ st1,
                                          char *__restrict__ st2, char *__restrict__ st3, const uint16_t *A,
-                                         const uint16_t *B, int64_t krange, int ntiles, f32x16 (&acc)[FA][FB],
-                                         int wave, int lane) {
+                                         const uint16_t *B, int64_t rows_a, int64_t rows_b, int64_t krange, int ntiles,
+                                         f32x16 (&acc)[FA][FB], int wave, int lane) {
     // OPAQUE: the direct loads' LDS addresses hidden from the compiler (needed whenever the
     // stages share one LDS object or are three or more: then only the explicit waits order the
     // loads). FA / FB: 32-row A / 32-column B fragments per wave. FA = 4, FB = 4: 256 x 256 tile,
@@ -960,8 +965,8 @@ __device__ __forceinline__ void dtl_tile(const GemmArgs &p, char *__restrict__ s
     if (ntiles <= 0) return;
     OA oa;
     OB ob;
-    oa.init(A, p.lda, krange, wave, lane);
-    ob.init(B, p.ldb, krange, wave, lane, DUAL && wave >= 2 ? BN / 2 : 0);
+    oa.init(A, p.lda, EDGE ? rows_a : FA * 64, krange, wave, lane);
+    ob.init(B, p.ldb, EDGE ? rows_b : BN, krange, wave, lane, DUAL && wave >= 2 ? BN / 2 : 0);
     const int last = ntiles - 1;
     auto issue = [&](int t, char *stage) {
         const int64_t kk = (int64_t)min(t, last) * BK;
@@ -1090,7 +1095,7 @@ __device__ __forceinline__ void dtl_tile(const GemmArgs &p, char *__restrict__ s
 // write instruction touches (4 apart) then fall in different banks. In the SwiGLU form the gate
 // wave (wn = 0) and the up wave (wn = 1) of a row half stage the same output columns and then
 // finish 64 rows each of the pair.
-template <bool DUAL, int FB, int FA = 4>
+template <bool DUAL, int FB, int FA, bool EDGE>
 __device__ __forceinline__ void dtl_epilogue(const GemmArgs &p, char *st0, char *st1, char *st2,
                                              const f32x16 (&acc)[FA][FB], int64_t m0, int64_t n0, int64_t coff,
                                              int64_t z, int wave, int lane) {
@@ -1180,17 +1185,22 @@ __device__ __forceinline__ void dtl_epilogue(const GemmArgs &p, char *st0, char 
             }
         } else {
             const int64_t col = n0 + wn * (FB * 32) + hp * EC2 + cl;
+            // a tile that passes the last row or column
+            const bool edge = EDGE && (m0 + 2 * WT > p.M || n0 + FB * 64 > p.N);
             auto staged = [&](int h, int it) {
                 return *(const f32x4 *)((h ? hi : lo) + (4 * it + (lane >> 4)) * EP2 + ((cl ^ ((it & 1) << 5)) * 4));
             };
 #pragma unroll
             for (int h = 0; h < NH; ++h) {
                 const int64_t row0 = m0 + wm * WT + h * 64 + (lane >> 4);
-                if (p.splits > 1) {
+                if (edge) {
+#pragma unroll 4
+                    for (int it = 0; it < 16; ++it) finish4<true>(p, staged(h, it), row0 + 4 * it, col, coff, z);
+                } else if (p.splits > 1) {
                     // split-K partial sums: plain f32 rows of N
                     float *dst = p.partial + (z * p.M + row0) * p.N + col;
 #pragma unroll 4
-                    for (int it = 0; it < 16; ++it, dst += 4 * p.N) *(f32x4 *)dst = staged(h, it);
+                    for (int it = 0; it < 16; ++it, dst += 4 * p.N) *(f32x4_any *)dst = staged(h, it);
                 } else if (p.c_vec_ok && !p.row_scale && p.beta == 0.f && !p.rope_table) {
                     // the common epilogue: alpha (and a column bias) only, with one base pointer per half
                     f32x4 bias = {0.f, 0.f, 0.f, 0.f};
@@ -1201,12 +1211,12 @@ __device__ __forceinline__ void dtl_epilogue(const GemmArgs &p, char *st0, char 
 #pragma unroll 4
                         for (int it = 0; it < 16; ++it, dst += 4 * p.ldc) {
                             const f32x4 v = staged(h, it) * p.alpha + bias;
-                            *(u32x2 *)dst = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+                            *(u32x2_any *)dst = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
                         }
                     } else {
                         float *dst = (float *)p.C + idx;
 #pragma unroll 4
-                        for (int it = 0; it < 16; ++it, dst += 4 * p.ldc) *(f32x4 *)dst = staged(h, it) * p.alpha + bias;
+                        for (int it = 0; it < 16; ++it, dst += 4 * p.ldc) *(f32x4_any *)dst = staged(h, it) * p.alpha + bias;
                     }
                 } else {
 #pragma unroll 4
@@ -1225,7 +1235,7 @@ __device__ __forceinline__ void dtl_epilogue(const GemmArgs &p, char *st0, char 
 // accumulate gate and wn = 1 up for one 256 x 128 output tile; the epilogue pairs them. FB = 2:
 // a 256 x 128 output tile (twice the tiles where 256 x 256 would leave CUs idle), with three
 // stages of 48 KB.
-template <bool TA, bool TB, bool DUAL, int FB, bool OPAQUE = (FB == 2), int FA = 4, int NS = 0>
+template <bool TA, bool TB, bool DUAL, int FB, bool EDGE, bool OPAQUE = (FB == 2), int FA = 4, int NS = 0>
 __device__ __forceinline__ void dtl_block(const GemmArgs &p, int tile, int64_t z, char *st0, char *st1, char *st2,
                                           char *st3 = nullptr) {
     static_assert(!DUAL || (!TA && TB), "SwiGLU is Y = X.W^T");
@@ -1244,19 +1254,19 @@ __device__ __forceinline__ void dtl_block(const GemmArgs &p, int tile, int64_t z
     const T *Bm = (const T *)(DUAL && wave >= 2 ? p.B2 : p.B);
     const T *B = Bm + bo * p.sB_out + bi * p.sB_in + (TB ? n0 * p.ldb + kb : kb * p.ldb + n0);
     f32x16 acc[F][FB];
-    dtl_tile<TA, TB, DUAL, FB, OPAQUE, FA, NS>(p, st0, st1, st2, st3, A, B, ke - kb,
-                                               ke > kb ? (int)((ke - kb) / BK) : 0, acc, wave, lane);
-    dtl_epilogue<DUAL, FB, FA>(p, st0, st1, st2, acc, m0, n0, bo * p.sC_out + bi * p.sC_in, z, wave, lane);
+    dtl_tile<TA, TB, DUAL, FB, EDGE, OPAQUE, FA, NS>(p, st0, st1, st2, st3, A, B, p.M - m0, p.N - n0, ke - kb,
+                                                     ke > kb ? (int)((ke - kb) / BK) : 0, acc, wave, lane);
+    dtl_epilogue<DUAL, FB, FA, EDGE>(p, st0, st1, st2, acc, m0, n0, bo * p.sC_out + bi * p.sC_in, z, wave, lane);
 }
 
-template <bool TA, bool TB, bool DUAL = false, int FB = 4>
+template <bool TA, bool TB, bool DUAL = false, int FB = 4, bool EDGE = false>
 __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_bf16_dtl(const GemmArgs p) {
     constexpr int STAGE = (256 + (FB == 4 ? 256 : 128)) * 64 * 2;
     __shared__ __attribute__((aligned(1024))) char st0[STAGE];
     __shared__ __attribute__((aligned(1024))) char st1[STAGE];
     __shared__ __attribute__((aligned(1024))) char st2[FB == 2 ? STAGE : 16];  // FB = 2 only
-    dtl_block<TA, TB, DUAL, FB>(p, blockIdx.x, blockIdx.y, st0, st1, st2);
+    dtl_block<TA, TB, DUAL, FB, EDGE>(p, blockIdx.x, blockIdx.y, st0, st1, st2);
 }
 
 // 128 x 128 tiles (64 x 64 per wave), four stages of 32 KB: for shapes whose 256-wide tiles would
@@ -1265,7 +1275,7 @@ void gemm_bf16_dtl(const GemmArgs p) {
 // direct load (vmcnt(0)) before each transposing fragment read (ds_read_b64_tr_b16), so the loads
 // of an mn-contiguous operand never ran ahead of the k-tile being multiplied.
 constexpr int DTL128_STAGES = 4;
-template <bool TA, bool TB>
+template <bool TA, bool TB, bool EDGE>
 __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_bf16_dtl128(const GemmArgs p) {
     constexpr int STAGE = 2 * 128 * 64 * 2;
@@ -1274,7 +1284,7 @@ void gemm_bf16_dtl128(const GemmArgs p) {
     __shared__ __attribute__((aligned(1024))) char st1[STAGE];
     __shared__ __attribute__((aligned(1024))) char st2[STAGE];
     __shared__ __attribute__((aligned(1024))) char st3[STAGE];
-    dtl_block<TA, TB, false, 2, true, 2, DTL128_STAGES>(p, blockIdx.x, blockIdx.y, st0, st1, st2, st3);
+    dtl_block<TA, TB, false, 2, EDGE, true, 2, DTL128_STAGES>(p, blockIdx.x, blockIdx.y, st0, st1, st2, st3);
 }
 
 // BF16: 256 x 256 direct-to-LDS tiles, batch 1, no split-K, one round of CUs.
@@ -1286,7 +1296,7 @@ void gemm_bf16_dtl_group(const GemmGroupArgs grp) {
     __shared__ __attribute__((aligned(1024))) char st1[STAGE];
     int gi, split, tile;
     if (!group_block(grp, gi, split, tile)) return;
-    dtl_block<TA, TB, false, 4>(grp.g[gi], tile, 0, st0, st1, st0);
+    dtl_block<TA, TB, false, 4, false>(grp.g[gi], tile, 0, st0, st1, st0);
 }
 
 // FP32: 64 x 64 tiles, batch 1, one split count for the group. Split-K partial sums go to each
@@ -1383,29 +1393,41 @@ bool dtl128_applicable(bool ta, bool tb, const GemmArgs &a) {
            fits(!ta, a.lda) && fits(tb, a.ldb) && a.K * 2 < (1ll << 31);
 }
 
+template <bool EDGE>
 hipError_t launch_bf16_dtl128(bool ta, bool tb, const GemmArgs &a, dim3 grid, hipStream_t s) {
-    if (!ta && tb) hipLaunchKernelGGL((gemm_bf16_dtl128<false, true>), grid, dim3(NTHREADS), 0, s, a);
-    else if (!ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl128<false, false>), grid, dim3(NTHREADS), 0, s, a);
-    else if (ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl128<true, false>), grid, dim3(NTHREADS), 0, s, a);
-    else hipLaunchKernelGGL((gemm_bf16_dtl128<true, true>), grid, dim3(NTHREADS), 0, s, a);
+    if (!ta && tb) hipLaunchKernelGGL((gemm_bf16_dtl128<false, true, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+    else if (!ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl128<false, false, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+    else if (ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl128<true, false, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+    else hipLaunchKernelGGL((gemm_bf16_dtl128<true, true, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+    return hipGetLastError();
+}
+
+// The direct-to-LDS kernel of a plain product's bm x bn tile.
+template <bool EDGE>
+hipError_t launch_dtl(bool ta, bool tb, int bm, int bn, const GemmArgs &a, dim3 grid, hipStream_t s) {
+    if (bm == 128) return launch_bf16_dtl128<EDGE>(ta, tb, a, grid, s);
+    if (bn == 128) {
+        if (!ta && tb) hipLaunchKernelGGL((gemm_bf16_dtl<false, true, false, 2, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+        else if (!ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl<false, false, false, 2, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+        else if (ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl<true, false, false, 2, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+        else hipLaunchKernelGGL((gemm_bf16_dtl<true, true, false, 2, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+    } else {
+        if (!ta && tb) hipLaunchKernelGGL((gemm_bf16_dtl<false, true, false, 4, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+        else if (!ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl<false, false, false, 4, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+        else if (ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl<true, false, false, 4, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+        else hipLaunchKernelGGL((gemm_bf16_dtl<true, true, false, 4, EDGE>), grid, dim3(NTHREADS), 0, s, a);
+    }
     return hipGetLastError();
 }
 
 hipError_t launch_bf16_256(bool ta, bool tb, int bn, const GemmArgs &a, dim3 grid, hipStream_t s) {
     if (bn == 128) {  // the planner offers 256 x 128 only where the direct-to-LDS kernel applies
         if (!dtl_applicable(ta, tb, a, 128)) return hipErrorInvalidConfiguration;
-        if (!ta && tb) hipLaunchKernelGGL((gemm_bf16_dtl<false, true, false, 2>), grid, dim3(NTHREADS), 0, s, a);
-        else if (!ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl<false, false, false, 2>), grid, dim3(NTHREADS), 0, s, a);
-        else if (ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl<true, false, false, 2>), grid, dim3(NTHREADS), 0, s, a);
-        else hipLaunchKernelGGL((gemm_bf16_dtl<true, true, false, 2>), grid, dim3(NTHREADS), 0, s, a);
-        return hipGetLastError();
+        return launch_dtl<false>(ta, tb, 256, 128, a, grid, s);
     }
     if (dtl_applicable(ta, tb, a)) {
-        if (a.dual) hipLaunchKernelGGL((gemm_bf16_dtl<false, true, true>), grid, dim3(NTHREADS), 0, s, a);
-        else if (!ta && tb) hipLaunchKernelGGL((gemm_bf16_dtl<false, true>), grid, dim3(NTHREADS), 0, s, a);
-        else if (!ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl<false, false>), grid, dim3(NTHREADS), 0, s, a);
-        else if (ta && !tb) hipLaunchKernelGGL((gemm_bf16_dtl<true, false>), grid, dim3(NTHREADS), 0, s, a);
-        else hipLaunchKernelGGL((gemm_bf16_dtl<true, true>), grid, dim3(NTHREADS), 0, s, a);
+        if (!a.dual) return launch_dtl<false>(ta, tb, 256, 256, a, grid, s);
+        hipLaunchKernelGGL((gemm_bf16_dtl<false, true, true>), grid, dim3(NTHREADS), 0, s, a);
         return hipGetLastError();
     }
     if (tiles_exact(a, 256, a.dual ? 128 : 256, ET<uint16_t>::BK))
@@ -1676,6 +1698,179 @@ Plan choose_plan(const GemmArgs &a, bool bf16, int64_t cus, bool ta, bool tb, do
 
 }  // namespace
 
+namespace {
+
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+
+// One operand of a padded copy: BF16 [rows, cols] (leading dimension ld, any alignment) into
+// [rows_p, dst_ld], whose columns past `cols` and rows past `rows` are zeros.
+struct PadSide {
+    const uint16_t *src;
+    int64_t s_in, s_out, ld;
+    uint16_t *dst;
+    uint32_t rows, cols, rows_p, vecs;  // vecs = dst_ld / 8
+};
+struct PadArgs {
+    PadSide side[2];
+    int64_t inner;
+};
+
+// Both operands' copies in one launch (blockIdx.z: the side; blockIdx.y: the batch), 8 columns per
+// thread in one load of any alignment: 9 us for 1999 x 1237 and 3001 x 1237, against 16 us as two
+// launches of element loads.
+__global__ __launch_bounds__(256) void pad_bf16(const PadArgs p) {
+    const PadSide o = p.side[blockIdx.z];
+    const int64_t b = blockIdx.y;
+    const uint16_t *src = o.src + b / p.inner * o.s_out + b % p.inner * o.s_in;
+    uint16_t *dst = o.dst + b * o.rows_p * o.vecs * 8;
+    const uint32_t total = o.rows_p * o.vecs;  // the copies take at most 1 GB
+    for (uint32_t e = blockIdx.x * 256 + threadIdx.x; e < total; e += gridDim.x * 256) {
+        const uint32_t r = e / o.vecs, c = (e - r * o.vecs) * 8;
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (r < o.rows) {
+            const uint16_t *at = src + r * o.ld + c;
+            if (c + 8 <= o.cols) {
+                v = *(const u32x4_any *)at;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (c + i < o.cols) v[i >> 1] |= (uint32_t)at[i] << ((i & 1) * 16);
+            }
+        }
+        *(u32x4 *)(dst + (int64_t)e * 8) = v;
+    }
+}
+
+// A plain BF16 product that no whole-tile kernel takes, on the direct-to-LDS tiles: operands they can
+// read in place (16-byte aligned rows, K a multiple of 128) stay, others are copied into padded scratch
+// first, and edge tiles finish with bounds checks.
+struct Ragged {
+    Plan plan;
+    bool copy_a, copy_b;
+    int64_t kp, rows_a, ld_a, rows_b, ld_b;  // K padded; the copies' shapes (stored layout)
+    size_t bytes_a, bytes_b, bytes_part;     // scratch: the copies and the split-K partial sums
+};
+
+size_t align256(size_t n) { return (n + 255) / 256 * 256; }
+
+// False where the product is another kernel's or the ordinary plan is priced lower. That plan's price is
+// corrected for its loads at such sizes: measured 57 TFLOP/s element by element (1999 x 3001 x 1237) and
+// 265 with masked vectors (2000 x 3000 x 1240) where the model says about 250 and 420; the copies cost
+// 3 us and their traffic at 2.5 TB/s.
+// plain, t_plain: the ordinary plan and its estimate.
+bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &plain, double t_plain, Ragged &r) {
+    constexpr int bk = ET<uint16_t>::BK;
+    if (a.M % 128 == 0 && a.N % 128 == 0 && a.K % 128 == 0 && a.a_vec_ok && a.b_vec_ok) return false;
+    if (a.dual || a.causal != CAUSAL_NONE || a.kmode != KMODE_FULL || a.swiglu_bwd || a.xent_stats || a.a_kscale ||
+        a.rope_table || a.K < 64 || a.M < 64 || a.N < 64 || a.batch > 65535)
+        return false;
+    GemmArgs d = a;
+    d.k_per_split = plain.k_per_split > 0 ? plain.k_per_split : cdiv(cdiv(a.K, plain.splits), bk) * bk;
+    if (plain.bm == 256 ? dtl_applicable(ta, tb, d, plain.bn) : plain.bm == 128 && dtl128_applicable(ta, tb, d))
+        return false;
+    const bool vectors = vectors_exact<uint16_t>(a, ta, tb);
+    if (!tiles_exact(d, plain.bm, plain.bn, bk)) t_plain *= vectors && plain.bm != 256 ? 1.6 : 4.0;
+
+    r.kp = cdiv(a.K, 128) * 128;
+    r.copy_a = !a.a_vec_ok || r.kp != a.K;
+    r.copy_b = !a.b_vec_ok || r.kp != a.K;
+    r.rows_a = ta ? r.kp : a.M;
+    r.ld_a = ta ? cdiv(a.M, 8) * 8 : r.kp;
+    r.rows_b = tb ? a.N : r.kp;
+    r.ld_b = tb ? r.kp : cdiv(a.N, 8) * 8;
+    r.bytes_a = r.copy_a ? align256((size_t)a.batch * r.rows_a * r.ld_a * 2) : 0;
+    r.bytes_b = r.copy_b ? align256((size_t)a.batch * r.rows_b * r.ld_b * 2) : 0;
+    const double copies = ((r.copy_a || r.copy_b) ? 3e-6 : 0.0) + 2.0 * (r.bytes_a + r.bytes_b) / 2.5e12;
+    double best = 1e30;
+    for (const int unit : {256, 128}) {  // whole tiles of this unit cover the product
+        GemmArgs e = a;
+        e.M = cdiv(a.M, unit) * unit;
+        e.N = cdiv(a.N, unit) * unit;
+        e.K = r.kp;
+        if (r.copy_a) e.lda = r.ld_a;
+        if (r.copy_b) e.ldb = r.ld_b;
+        e.a_vec_ok = e.b_vec_ok = 1;
+        double t = 0.0;
+        Plan pl = choose_plan(e, true, cus, ta, tb, &t);
+        if (plain.bm == 256 && plain.splits > 1) pl = Plan{256, 256, plain.splits, 0};  // as its price is compared
+        if (pl.k_per_split <= 0) pl.k_per_split = cdiv(cdiv(e.K, pl.splits), 128) * 128;
+        e.k_per_split = pl.k_per_split;
+        bool dtl = pl.bm == 256 ? dtl_applicable(ta, tb, e, pl.bn) : pl.bm == 128 && dtl128_applicable(ta, tb, e);
+        if (!dtl) {  // the register-staged tiles are priced lower there: one 128 x 128 tile per CU
+            pl = Plan{128, 128, 1, e.K};
+            e.k_per_split = e.K;
+            t = cdiv(cdiv(a.M, 128) * cdiv(a.N, 128) * a.batch, cus) * (3e-6 + e.K / 64 * 0.56e-6);
+            dtl = dtl128_applicable(ta, tb, e);
+        }
+        if (dtl && t < best) {
+            best = t;
+            r.plan = pl;
+        }
+    }
+    r.bytes_part = r.plan.splits > 1 ? (size_t)r.plan.splits * a.batch * a.M * a.N * sizeof(float) : 0;
+    return best + copies < t_plain && r.bytes_a + r.bytes_b <= (size_t(1) << 30);
+}
+
+// Whether the scratch can be had now: a capture may not allocate.
+bool scratch_ready(const it_context *ctx, size_t bytes) {
+    return !ctx->capturing || ctx->scratch_bytes[ctx->cur] >= bytes;
+}
+
+it_status launch_ragged(it_context *ctx, bool ta, bool tb, GemmArgs a, const Ragged &r, void *ws, const char *tag) {
+    std::string key;
+    hipEvent_t ev = nullptr;
+    if (ctx->profiling) {
+        char buf[192];
+        std::snprintf(buf, sizeof(buf), "gemm_bf16_%c%c_%dx%d_dtl_edge|%s[%lld,%lld,%lld]x%lld s%d", ta ? 'T' : 'N',
+                      tb ? 'T' : 'N', r.plan.bm, r.plan.bn, tag ? tag : "", (long long)a.M, (long long)a.N,
+                      (long long)a.K, (long long)a.batch, r.plan.splits);
+        key = buf;
+        profile_begin(ctx, key, &ev);
+    }
+    PadArgs pad{};
+    pad.inner = a.batch_inner;
+    int sides = 0;
+    int64_t most = 0;  // 16-byte vectors of the larger copy
+    char *at = (char *)ws;
+    auto copy = [&](const void *&src, int64_t &s_in, int64_t &s_out, int64_t &ld, int64_t rows, int64_t cols,
+                    int64_t rows_p, int64_t dst_ld, size_t bytes) {
+        pad.side[sides++] = PadSide{(const uint16_t *)src, s_in, s_out, ld, (uint16_t *)at, (uint32_t)rows,
+                                    (uint32_t)cols, (uint32_t)rows_p, (uint32_t)(dst_ld / 8)};
+        most = std::max(most, rows_p * (dst_ld / 8));
+        src = at;
+        ld = dst_ld;
+        s_in = rows_p * dst_ld;
+        s_out = a.batch_inner * s_in;
+        at += bytes;
+    };
+    if (r.copy_a)
+        copy(a.A, a.sA_in, a.sA_out, a.lda, ta ? a.K : a.M, ta ? a.M : a.K, r.rows_a, r.ld_a, r.bytes_a);
+    if (r.copy_b)
+        copy(a.B, a.sB_in, a.sB_out, a.ldb, tb ? a.N : a.K, tb ? a.K : a.N, r.rows_b, r.ld_b, r.bytes_b);
+    if (sides) {
+        const dim3 grid((unsigned)std::min<int64_t>(cdiv(most, 256), 8192), (unsigned)a.batch, (unsigned)sides);
+        hipLaunchKernelGGL(pad_bf16, grid, dim3(256), 0, ctx->stream, pad);
+    }
+    a.partial = (float *)at;
+    a.K = r.kp;
+    a.a_vec_ok = a.b_vec_ok = a.c_vec_ok = 1;  // C: 4-column vectors of any alignment
+    a.tiles_m = (int)cdiv(a.M, r.plan.bm);
+    a.tiles_n = (int)cdiv(a.N, r.plan.bn);
+    a.k_per_split = r.plan.k_per_split;
+    a.splits = (int)cdiv(a.K, a.k_per_split);
+    const dim3 grid((unsigned)(a.tiles_m * a.tiles_n), (unsigned)(a.batch * a.splits));
+    const hipError_t e = launch_dtl<true>(ta, tb, r.plan.bm, r.plan.bn, a, grid, ctx->stream);
+    if (e != hipSuccess) return fail_hip(e, "gemm_bf16_dtl launch");
+    if (a.splits > 1) {
+        const it_status st = launch_splitk_reduce(ctx->stream, a);
+        if (st != IT_OK) return st;
+    }
+    if (ctx->profiling) profile_end(ctx, key, ev);
+    return IT_OK;
+}
+
+}  // namespace
+
 it_status launch_splitk_reduce(hipStream_t s, const GemmArgs &a) {
     const int64_t total = a.batch * a.M * a.N;
     if (a.N % 4 == 0) {
@@ -1741,7 +1936,15 @@ it_status launch_gemm(it_context *ctx, it_dtype dtype_in, bool transA, bool tran
     if (!bf16 && f32_terms_applicable(a, transA, transB)) return launch_gemm_f32(ctx, transA, transB, a, profile_tag);
     const int bk = bf16 ? ET<uint16_t>::BK : ET<float>::BK;
     const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-    Plan plan = choose_plan(a, bf16, cus, transA, transB);
+    double t_plan = 0.0;
+    Plan plan = choose_plan(a, bf16, cus, transA, transB, &t_plan);
+    if (Ragged r; bf16 && plan_ragged(a, cus, transA, transB, plan, t_plan, r)) {
+        const size_t bytes = r.bytes_a + r.bytes_b + r.bytes_part;
+        void *ws = nullptr;
+        if (a.batch * r.plan.splits <= 65535 && scratch_ready(ctx, bytes) &&
+            (bytes == 0 || ensure_scratch(ctx, bytes, &ws) == IT_OK))
+            return launch_ragged(ctx, transA, transB, a, r, ws, profile_tag);
+    }
 #ifdef IT_TUNING
     // Planner sweeps only (a tuning build): IT_PLAN="tile,splits[,width]" forces the plan.
     if (const char *env = std::getenv("IT_PLAN")) {
@@ -1796,7 +1999,7 @@ it_status launch_gemm(it_context *ctx, it_dtype dtype_in, bool transA, bool tran
         profile_begin(ctx, key, &ev);
     }
     hipError_t e = bf16 && cfg.bm == 256 ? launch_bf16_256(transA, transB, a.dual ? 256 : cfg.bn, a, grid, ctx->stream)
-                   : dtl128      ? launch_bf16_dtl128(transA, transB, a, grid, ctx->stream)
+                   : dtl128      ? launch_bf16_dtl128<false>(transA, transB, a, grid, ctx->stream)
                    : bf16        ? launch_typed<uint16_t>(transA, transB, a.dual, cfg, a, grid, ctx->stream)
                                  : launch_typed<float>(transA, transB, a.dual, cfg, a, grid, ctx->stream);
     if (e != hipSuccess) return fail_hip(e, "gemm_mfma launch");

@@ -654,6 +654,11 @@ bool f32_terms_applicable(const GemmArgs &a, bool ta, bool tb) {
 
 it_status launch_gemm_f32(it_context *ctx, bool ta, bool tb, GemmArgs a, const char *tag) {
     Plan plan = choose_plan(a, cus_of(ctx), ta, nullptr);
+    if (plan.splits > 1 && ctx->capturing &&
+        ctx->scratch_bytes[ctx->cur] < (size_t)plan.splits * a.batch * a.M * a.N * sizeof(float)) {
+        a.no_split = 1;  // a capture may not allocate
+        plan = choose_plan(a, cus_of(ctx), ta, nullptr);
+    }
 #ifdef IT_TUNING
     // Planner sweeps only (a tuning build): IT_PLAN="tile,splits[,width]" forces the plan.
     if (const char *env = std::getenv("IT_PLAN")) {
@@ -790,6 +795,9 @@ bool launch_gemm_f32_group(it_context *ctx, bool ta, bool tb, const GemmArgs *ar
     const int grid_blocks = xcd_schedule(grp);
     if (!grid_blocks) return false;
     if (split_any) {
+        if (ctx->capturing &&
+            (!ctx->counters[ctx->cur] || ctx->scratch_bytes[ctx->cur] < (size_t)scratch * sizeof(float)))
+            return false;  // a capture may not allocate
         *status = ensure_counters(ctx, &grp.arrive);
         if (*status != IT_OK) return true;
         void *ws = nullptr;
