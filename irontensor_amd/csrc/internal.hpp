@@ -220,9 +220,10 @@ struct FlashArgs {
     float scale;
     int causal;
 };
-// Decode-shaped BF16 NT GEMM (M <= 16), HBM-bound: kernels_gemv.hip.
+// Decode-shaped NT GEMM (M <= 16), BF16 or FP32, HBM-bound: kernels_gemv.hip.
 bool gemv_applicable(const GemmArgs &a, bool bf16, bool transA, bool transB);
-it_status launch_gemv(hipStream_t s, const GemmArgs &a);
+bool gemv_f32_applicable(const GemmArgs &a, bool transA, bool transB);
+it_status launch_gemv(hipStream_t s, bool bf16, const GemmArgs &a);
 // Decode-shaped BF16 GEMM with the weight stored [K, N] (NN, and TN with X stored [K, M]), M <= 16:
 // gemv_kn_splits picks the k splits; with more than one, a.partial must hold
 // splits * batch * M * N floats and `counters` one zero int per (column strip, batch item).

@@ -649,6 +649,7 @@ void any_alignment(GemmArgs &a) { a.c_vec_ok = a.c_vec_ok || !a.out_bf16; }
 bool f32_terms_applicable(const GemmArgs &a, bool ta, bool tb) {
     // A few rows wait on latency, not on the matrix units: M = 1, N = 768, K = 256 takes 6.7 us here
     // and 6.0 on the FP32 units' 64 x 32 tile, which loads two k-tiles ahead.
+    // (X.W^T there goes to gemv_nt where its rows are whole 16-byte chunks.)
     return a.M > 16 && !a.f32_units && !a.a_kscale && !a.xent_stats && spans_fit(a, ta, tb);
 }
 

@@ -22,6 +22,9 @@
 // Measured at K 4096, N 11008 with cold weights: 18.7 / 19.8 / 20.6 us at M = 1 / 4 / 16 (the direct
 // layout: 20.6 / 22.0 / 28.3 us). Two or four column blocks per wave sharing the X fragments
 // measured slower: half or a quarter of the blocks.
+//
+// FP32 operands run the same kernel with 4-element chunks (a pair of loads covers 32 k) on
+// v_mfma_f32_16x16x4_f32, whose rate is four times what the weight stream needs at M = 16.
 #include <algorithm>
 
 #include "epilogue.hpp"
@@ -32,8 +35,7 @@ namespace it {
 namespace {
 
 constexpr int GV_THREADS = 256;
-constexpr int GV_UNROLL = 8;   // 32-wide k chunks per wave per iteration (4 pairs of loads)
-constexpr int GV_KCHUNK = 32;
+constexpr int GV_UNROLL = 8;  // operand fragments (64 bytes of a row) per wave per iteration: 4 pairs of loads
 
 // Weights are streamed once per call. The [K, N] kernel loads them nontemporally (measured 4-8%
 // faster with cold weights); the [N, K] kernel measured 2-4% slower that way and loads them plainly.
@@ -52,9 +54,11 @@ constexpr uint32_t GV_OOB = 0x80000000u;
 __device__ __forceinline__ int gv_slot(int rr, int c) { return rr * 8 + (c ^ rr); }
 
 // XHI: M > 8, so X rows 8-15 are loaded too (otherwise MFMA rows 8-15 of X repeat rows 0-7; they
-// only reach output rows past M, which are not written).
-template <bool XHI>
-__global__ __launch_bounds__(GV_THREADS) void gemv_bf16_nt(const GemmArgs p) {
+// only reach output rows past M, which are not written). T: uint16_t (BF16) or float.
+template <typename T, bool XHI>
+__global__ __launch_bounds__(GV_THREADS) void gemv_nt(const GemmArgs p) {
+    constexpr int EB = sizeof(T), EC = 16 / EB;  // bytes per element, elements per 16-byte chunk
+    constexpr int KCHUNK = 4 * EC;               // k of one operand fragment
     // Per wave: two slots (pairs alternate), each W rows 0-7, W rows 8-15, X rows 0-7, X rows 8-15.
     __shared__ u32x4 stage[4][2][4][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -63,8 +67,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_bf16_nt(const GemmArgs p) {
     const int64_t n0 = (int64_t)blockIdx.x * 16;
     const int64_t z = blockIdx.y;
     const int64_t bo = z / p.batch_inner, bi = z % p.batch_inner;
-    const uint16_t *X = (const uint16_t *)p.A + bo * p.sA_out + bi * p.sA_in;
-    const uint16_t *W = (const uint16_t *)p.B + bo * p.sB_out + bi * p.sB_in + n0 * p.ldb;
+    const T *X = (const T *)p.A + bo * p.sA_out + bi * p.sA_in;
+    const T *W = (const T *)p.B + bo * p.sB_out + bi * p.sB_in + n0 * p.ldb;
     const int64_t coff = bo * p.sC_out + bi * p.sC_in;
 
     // Buffer descriptors over exactly the block's W rows and X's M rows (byte extents below 2^31,
@@ -72,30 +76,30 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_bf16_nt(const GemmArgs p) {
     // read as zeros with no memory access.
     const int64_t nrows = min((int64_t)16, p.N - n0);
     const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t *>(W), (short)0, (int)(((nrows - 1) * p.ldb + p.K) * 2), 0x00020000);
+        const_cast<T *>(W), (short)0, (int)(((nrows - 1) * p.ldb + p.K) * EB), 0x00020000);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t *>(X), (short)0, (int)(((p.M - 1) * p.lda + p.K) * 2), 0x00020000);
-    const uint32_t wo0 = (uint32_t)(rl * p.ldb * 2), wo1 = (uint32_t)((8 + rl) * p.ldb * 2);
-    const uint32_t xo0 = (uint32_t)(rl * p.lda * 2), xo1 = (uint32_t)((8 + rl) * p.lda * 2);
+        const_cast<T *>(X), (short)0, (int)(((p.M - 1) * p.lda + p.K) * EB), 0x00020000);
+    const uint32_t wo0 = (uint32_t)(rl * p.ldb * EB), wo1 = (uint32_t)((8 + rl) * p.ldb * EB);
+    const uint32_t xo0 = (uint32_t)(rl * p.lda * EB), xo1 = (uint32_t)((8 + rl) * p.lda * EB);
     // LDS slots: where this lane's loaded chunk goes, and where its operand chunks come from.
     const int wslot = gv_slot(rl, kc);
     const int rq = r >> 3, rr = r & 7;
     const int lo_slot = gv_slot(rr, g), hi_slot = gv_slot(rr, 4 + g);
     const int xq = XHI ? rq : 0;
 
-    // K split over the 4 waves in multiples of the 32-wide chunk.
-    const int64_t span = ((p.K + 4 * GV_KCHUNK - 1) / (4 * GV_KCHUNK)) * GV_KCHUNK;
+    // K split over the 4 waves in multiples of a fragment.
+    const int64_t span = ((p.K + 4 * KCHUNK - 1) / (4 * KCHUNK)) * KCHUNK;
     const int64_t kb = wave * span, ke = min(p.K, kb + span);
 
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int64_t k = kb; k < ke; k += GV_UNROLL * GV_KCHUNK) {
+    for (int64_t k = kb; k < ke; k += GV_UNROLL * KCHUNK) {
         u32x4 wr[GV_UNROLL], xr[GV_UNROLL];
 #pragma unroll
         for (int pr = 0; pr < GV_UNROLL / 2; ++pr) {
-            // This lane's chunk: 8 elements, and K % 8 == 0, so a chunk is whole or past the end.
-            const int64_t kk = k + 64 * pr + 8 * kc;
+            // This lane's chunk: EC elements, and K % EC == 0, so a chunk is whole or past the end.
+            const int64_t kk = k + 8 * EC * pr + EC * kc;
             const bool ok = kk < ke;
-            const uint32_t ko = (uint32_t)(kk * 2);
+            const uint32_t ko = (uint32_t)(kk * EB);
             wr[2 * pr] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, ok ? wo0 + ko : GV_OOB, 0, 0));
             wr[2 * pr + 1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, ok ? wo1 + ko : GV_OOB, 0, 0));
             xr[2 * pr] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, ok ? xo0 + ko : GV_OOB, 0, 0));
@@ -118,8 +122,8 @@ __global__ __launch_bounds__(GV_THREADS) void gemv_bf16_nt(const GemmArgs p) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             const u32x4 wlo = st[rq][lo_slot], whi = st[rq][hi_slot];
             const u32x4 xlo = st[2 + xq][lo_slot], xhi = st[2 + xq][hi_slot];
-            mma16<uint16_t>(acc, xlo, wlo);
-            mma16<uint16_t>(acc, xhi, whi);
+            mma16<T>(acc, xlo, wlo);
+            mma16<T>(acc, xhi, whi);
         }
     }
     // acc: lane l holds column n0 + l%16 and rows 4*(l/16) + i.
@@ -386,12 +390,30 @@ bool gemv_applicable(const GemmArgs &a, bool bf16, bool transA, bool transB) {
            (a.N + 15) / 16 <= 0x7fffffff && a.batch <= 65535;
 }
 
-it_status launch_gemv(hipStream_t s, const GemmArgs &a) {
-    dim3 grid((unsigned)((a.N + 15) / 16), (unsigned)a.batch);
-    if (a.M > 8)
-        hipLaunchKernelGGL(gemv_bf16_nt<true>, grid, dim3(GV_THREADS), 0, s, a);
+// FP32 (X.W^T, M <= 16; the same 2^31 bound in FP32 elements). Against the 64 x 32 tile of the FP32 units,
+// which multiplies 64 rows whatever M is, M = 1 (weights in cache, us): K 688, N 256 10.3 -> 6.0, K 1024,
+// N 4096 13.2 -> 6.2, K 256, N 16384 8.2 -> 6.2, K 4096, N 11008 52.9 -> 28.7 (6.3 TB/s), and the same at
+// M = 16; K 256, N 768 6.6 -> 6.2 (a call's own cost). Error against 64 bits at that size 2.7e-7 -> 1.5e-7.
+// Products that ask for the FP32 units' sums in the tile's order (f32_units), and epilogues that this
+// kernel has not, keep the tiles.
+bool gemv_f32_applicable(const GemmArgs &a, bool transA, bool transB) {
+    return !transA && transB && a.M >= 1 && a.M <= 16 && a.K > 0 && a.K % 4 == 0 && !a.f32_units && !a.dual &&
+           a.causal == CAUSAL_NONE && a.kmode == KMODE_FULL && !a.swiglu_bwd && !a.xent_stats && !a.a_kscale &&
+           !a.row_scale && !a.rope_table && a.a_vec_ok && a.b_vec_ok && a.lda >= a.K && a.ldb >= a.K &&
+           16 * a.lda + a.K < (1ll << 29) && 16 * a.ldb + a.K < (1ll << 29) && (a.N + 15) / 16 <= 0x7fffffff &&
+           a.batch <= 65535;
+}
+
+it_status launch_gemv(hipStream_t s, bool bf16, const GemmArgs &a) {
+    const dim3 grid((unsigned)((a.N + 15) / 16), (unsigned)a.batch), block(GV_THREADS);
+    if (bf16 && a.M > 8)
+        hipLaunchKernelGGL((gemv_nt<uint16_t, true>), grid, block, 0, s, a);
+    else if (bf16)
+        hipLaunchKernelGGL((gemv_nt<uint16_t, false>), grid, block, 0, s, a);
+    else if (a.M > 8)
+        hipLaunchKernelGGL((gemv_nt<float, true>), grid, block, 0, s, a);
     else
-        hipLaunchKernelGGL(gemv_bf16_nt<false>, grid, dim3(GV_THREADS), 0, s, a);
+        hipLaunchKernelGGL((gemv_nt<float, false>), grid, block, 0, s, a);
     IT_HIP_TRY(hipGetLastError());
     return IT_OK;
 }
