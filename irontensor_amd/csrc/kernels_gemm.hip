@@ -380,12 +380,14 @@ __device__ __forceinline__ void gemm_mfma_block(const GemmArgs &p, int tile, int
     // Register staging sets: PF of them, so the loads of tile t+PF are issued during tile t.
     OA oa[PF];
     constexpr bool RSRC = LM == LOAD_RSRC;
-    static_assert(!RSRC || (sizeof(T) == 4 && !DUAL && !KS && !XF), "LOAD_RSRC: plain FP32 tiles");
+    static_assert(!RSRC || (sizeof(T) == 4 && !KS && !XF), "LOAD_RSRC: FP32 tiles without operand transforms");
     RsrcLoad<!TA, BM> ra;
-    RsrcLoad<TB, BN> rb;
+    RsrcLoad<TB, DUAL ? BN / 2 : BN> rb, rb2;  // rb2: DUAL's up weight, with its own end
     if constexpr (RSRC) {
+        const int64_t span_b = (TB ? (p.N - 1) * p.ldb + p.K : (p.K - 1) * p.ldb + p.N) * 4;
         ra.init((const float *)A, p.lda, m0, (TA ? (p.K - 1) * p.lda + p.M : (p.M - 1) * p.lda + p.K) * 4, tid);
-        rb.init((const float *)B, p.ldb, n0, (TB ? (p.N - 1) * p.ldb + p.K : (p.K - 1) * p.ldb + p.N) * 4, tid);
+        rb.init((const float *)B, p.ldb, n0, span_b, tid);
+        if constexpr (DUAL) rb2.init((const float *)B2, p.ldb, n0, span_b, tid);
     }
     // SwiGLU (DUAL): the B tile's rows 0..BN/2-1 are gate-weight rows and BN/2..BN-1 the same up-
     // weight rows, so waves wn = 0 / 1 accumulate gate / up of one BM x BN/2 output tile and the
@@ -399,6 +401,7 @@ __device__ __forceinline__ void gemm_mfma_block(const GemmArgs &p, int tile, int
                 if constexpr (RSRC) {
                     ra.load(oa[q], k0, tid);
                     rb.load(ob[q], k0, tid);
+                    if constexpr (DUAL) rb2.load(ob2[q], k0, tid);
                 } else {
                     oa[q].template load<LM>(A, p.lda, m0, k0, p.M, ke, p.a_vec_ok, tid);
                     if constexpr (KS) oa[q].load_kscale(p.a_kscale, k0, ke, tid);
@@ -1515,7 +1518,7 @@ bool rsrc_ok(const GemmArgs &a, bool ta, bool tb) {
            (ta ? a.K : a.M) * a.lda * 4 < (1ll << 31) && (tb ? a.N : a.K) * a.ldb * 4 < (1ll << 31);
 }
 
-// The load mode of a plain tile: exact, buffer-descriptor (FP32), masked or checked.
+// The load mode of a tile without operand transforms: exact, buffer-descriptor (FP32), masked or checked.
 template <typename T>
 int load_mode_for(const GemmArgs &a, bool ta, bool tb, int bm, int bn) {
     int mode = tiles_exact(a, bm, bn, ET<T>::BK)                        ? LOAD_EXACT
@@ -1536,15 +1539,12 @@ int load_mode_for(const GemmArgs &a, bool ta, bool tb, int bm, int bn) {
 template <typename T, bool TA, bool TB, bool DUAL>
 hipError_t launch_cfg(const TileCfg &cfg, const GemmArgs &a, dim3 grid, hipStream_t s) {
     // cfg.bn is the output tile's width: for SwiGLU already half of the B tile's rows.
-    const int mode = DUAL ? (tiles_exact(a, cfg.bm, cfg.bn, ET<T>::BK) ? LOAD_EXACT
-                             : vectors_exact<T>(a, TA, TB)              ? LOAD_MASKED
-                                                                        : LOAD_CHECKED)
-                          : load_mode_for<T>(a, TA, TB, cfg.bm, cfg.bn);
+    const int mode = load_mode_for<T>(a, TA, TB, cfg.bm, cfg.bn);
     if (mode == LOAD_EXACT)
         launch_cfg_lm<T, TA, TB, DUAL, LOAD_EXACT>(cfg, a, grid, s);
     else if (mode == LOAD_MASKED)
         launch_cfg_lm<T, TA, TB, DUAL, LOAD_MASKED>(cfg, a, grid, s);
-    else if constexpr (sizeof(T) == 4 && !DUAL) {
+    else if constexpr (sizeof(T) == 4) {
         if (mode == LOAD_RSRC)
             launch_cfg_lm<T, TA, TB, DUAL, LOAD_RSRC>(cfg, a, grid, s);
         else

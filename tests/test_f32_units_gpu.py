@@ -1,0 +1,54 @@
+"""FP32 products that ask for the FP32 units (IT_EPI_F32_UNITS, the training step's default): the tiles
+that other FP32 products reach only with few rows.
+
+Bound per element, against the float64 product of the same operands: K products and sums, each rounded
+once, in any order, so |error| <= (K + 2) 2^-24 (|A|.|B|)_ij.
+"""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from irontensor_amd import _lib, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _within(got, a, b, extra=0.0):
+    """a.b^T in float64 against got."""
+    A, B = a.astype(np.float64), b.astype(np.float64)
+    bound = (a.shape[1] + 2) * 2.0 ** -24 * (np.abs(A) @ np.abs(B).T) + 2.0 ** -23 * np.abs(extra)
+    worst = float(np.max(np.abs(got - (A @ B.T + extra)) / bound))
+    assert worst <= 1.0, f"error {worst:.2f} times its bound"
+
+
+@pytest.mark.parametrize("rows,h,f", [(65, 64, 52), (200, 256, 688), (4096, 256, 688), (130, 32, 36), (64, 96, 4),
+                                      (1000, 36, 700), (129, 35, 33), (256, 128, 2048)])
+def test_swiglu_weights_inside_nan(it, rows, h, f):
+    """Widths that no tile divides: the rows past X, past the gate and past the up weight are NaN and
+    reach no result. Descriptor loads where h is a multiple of 32 (200 x 256 x 688), masked and
+    bounds-checked ones elsewhere, plain ones on whole tiles."""
+    print(f"[units swiglu] {rows}x{h}x{f}", flush=True)
+    x, wg, wu = synth.normal(1, (rows, h)), synth.normal(2, (f, h), std=0.05), synth.normal(3, (f, h), std=0.05)
+    bias = synth.normal(4, (2 * f,), std=0.1)
+    gap = np.full((70, h), np.nan, np.float32)
+    X = it.Tensor.from_f32_slice(np.concatenate([x, gap]), [rows + 70, h])
+    W = it.Tensor.from_f32_slice(np.concatenate([gap, wg, gap, wu, gap]), [2 * f + 210, h])
+    Bias = it.Tensor.from_f32_slice(bias, [2 * f])
+    outs = [it.Tensor.from_f32_slice(np.full((rows + 2, f), 7.0, np.float32), [rows + 2, f]) for _ in range(3)]
+    inner = [t.ptr + 4 * f for t in outs]
+    epi = _lib.Epilogue(flags=_lib.IT_EPI_SWIGLU | _lib.IT_EPI_BIAS | _lib.IT_EPI_F32_UNITS, bias=Bias.ptr,
+                        B2=W.ptr + 4 * h * (f + 140), gate_out=inner[1], up_out=inner[2])
+    st = X.ctx.lib.it_gemm(X.ctx.handle, 0, 0, 0, 1, rows, f, h, 1.0, C.c_void_p(X.ptr), h, 0,
+                           C.c_void_p(W.ptr + 4 * h * 70), h, 0, 0.0, C.c_void_p(inner[0]), f, 0, 1, C.byref(epi))
+    assert st == 0
+    hh, g, u = (t.numpy() for t in outs)
+    for t in (hh, g, u):
+        assert np.all(t[0] == 7.0) and np.all(t[-1] == 7.0)
+    _within(g[1:-1], x, wg, bias[None, :f].astype(np.float64))
+    _within(u[1:-1], x, wu, bias[None, f:].astype(np.float64))
+    gate, up = g[1:-1].astype(np.float64), u[1:-1].astype(np.float64)
+    ref = gate / (1 + np.exp(-gate)) * up
+    assert np.max(np.abs(hh[1:-1] - ref)) <= 4e-6 * np.max(np.abs(ref))
