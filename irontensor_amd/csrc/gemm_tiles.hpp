@@ -129,7 +129,7 @@ __device__ __forceinline__ void map_tile(int pid, int tiles_m, int tiles_n, int 
 }
 
 namespace sg {
-constexpr int MFMA = 0x008, VMEM_READ = 0x020, DS_READ = 0x100, DS_WRITE = 0x200;
+constexpr int VALU = 0x002, MFMA = 0x008, VMEM_READ = 0x020, DS_READ = 0x100, DS_WRITE = 0x200;
 }
 
 constexpr int CP_DEVICE_SCOPE = 16;  // cache-policy bit sc1 of the buffer intrinsics: device scope

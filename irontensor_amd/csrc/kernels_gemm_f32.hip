@@ -16,7 +16,7 @@
 //   * v_mfma_f32_16x16x32_bf16 blocks (the 32x32x16 form measured 2-6% slower in these tiles);
 //   * one LDS stage and two barriers per k-tile (gemm_f32_block), so that several blocks share a CU;
 //   * an accumulator that is not finite is computed again on the FP32 units, since the terms of an
-//     infinity (or of a value that rounds up to 2^128) are NaN.
+//     infinity (or of a value that rounds up to 2^112: the terms are scaled) are NaN.
 #include <cstdio>
 #include <string>
 
@@ -350,7 +350,16 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
 #pragma unroll
                     for (int j = 0; j < FN; ++j) acc[i][j] += lo[j];
                 }
-                // Strips in order: left alone, the scheduler gathers all splits first and spills.
+                // Strips in order: left alone, the scheduler gathers all splits first and spills. The
+                // wide tiles' split runs between their MFMAs: 4096^3 679 -> 653 us (X.W^T); the 64 x 64
+                // tile measured 1% slower so.
+                if constexpr (S::WIDE) {
+#pragma unroll
+                    for (int g = 0; g < 6 * FN; ++g) {
+                        __builtin_amdgcn_sched_group_barrier(sg::VALU, 2, 0);
+                        __builtin_amdgcn_sched_group_barrier(sg::MFMA, 1, 0);
+                    }
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
@@ -398,8 +407,9 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
                     acc[i][j] += *(const f32x4 *)(smem0 + g * REGION + ((i * FN + j) * THREADS + tid) * 16);
     }
 
-    // An element that is not finite (acc * 0 is NaN) may owe that to the split: this wave then takes
-    // its products again on the FP32 units, straight from memory.
+    // The sums are of scaled terms (BF16X3_SCALE for each operand). An element that is not finite (acc * 0
+    // is NaN) may owe that to the split or to the scale: this wave then takes its products again on the
+    // FP32 units, straight from memory.
     // Lane l of a 16x16 block holds rows (XPOSE: columns) 4 (l / 16) + r, r = 0..3, and column (row)
     // l % 16.
     float nf = 0.f;
@@ -449,6 +459,11 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
                     acc[i][j] = XPOSE ? __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j], av[i], acc[i][j], 0, 0, 0)
                                       : __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
         }
+    } else {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] *= 1.f / (BF16X3_SCALE * BF16X3_SCALE);
     }
 
     if constexpr (XPOSE) {

@@ -28,16 +28,18 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 
-// Two FP32 values as three BF16 terms each, x = t0 + t1 + t2 (packed in pairs, the first value low):
-// every term is the round-to-nearest-even of what the terms before it leave, and those differences
-// are exact, so the terms carry 3 x 8 = 24 significand bits (down to BF16's smallest step, 2^-133:
-// values below 2^-110 lose bits under it). An infinity, a NaN or a value that rounds up to 2^128
+// Two FP32 values times 2^16 as three BF16 terms each, x 2^16 = t0 + t1 + t2 (packed in pairs, the first
+// value low): every term is the round-to-nearest-even of what the terms before it leave, and those
+// differences are exact, so the terms carry 3 x 8 = 24 significand bits. Without the scale the last term
+// of values below 2^-110 would fall under BF16's smallest step, 2^-133; with it every FP32 value, the
+// subnormal ones included, keeps all its bits. An infinity, a NaN or a value that rounds up to 2^112
 // gives a NaN term.
+constexpr float BF16X3_SCALE = 65536.f;
 struct Bf16x3 {
     uint32_t t[3];
 };
 __device__ __forceinline__ Bf16x3 split_bf16x3(uint32_t bits0, uint32_t bits1) {
-    float a = __uint_as_float(bits0), b = __uint_as_float(bits1);
+    float a = __uint_as_float(bits0) * BF16X3_SCALE, b = __uint_as_float(bits1) * BF16X3_SCALE;
     Bf16x3 r;
 #pragma unroll
     for (int p = 0; p < 3; ++p) {

@@ -131,3 +131,18 @@ def test_training_step_on_the_fp32_units_or_terms(it):
         grads.append([t.numpy().astype(np.float64) for t in st.grads])
     for x, y in zip(*grads):
         assert np.linalg.norm(x - y) <= 2e-5 * np.linalg.norm(x)
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", [(70, 66, 80), (192, 200, 40), (640, 1152, 96), (512, 300, 4096)])
+@pytest.mark.parametrize("a_exp,b_exp", [(-110, 90), (-118, 100), (-126, 100), (-140, 120), (100, -125), (113, -60),
+                                         (70, 30)])
+def test_small_and_large_operands(it, ta, tb, m, n, k, a_exp, b_exp):
+    """Operands near either end of FP32's range keep their 24 bits: below 2^-110 the last of three unscaled
+    terms would lose its own (2^-126: all but 8 bits of an element), and subnormal operands have no more
+    bits than they show. Elements of 2^113 or sums above 2^96 leave the scaled terms' range."""
+    a, b = _operands(3, m, n, k, ta, tb)
+    a, b = np.ldexp(a, a_exp).astype(np.float32), np.ldexp(b / np.float32(0.02), b_exp).astype(np.float32)
+    c = it.gemm(it.Tensor.from_f32_slice(a, a.shape), it.Tensor.from_f32_slice(b, b.shape), trans_a=bool(ta),
+                trans_b=bool(tb))
+    _check(c.numpy(), a, b, ta, tb, k)
