@@ -206,7 +206,7 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
     using OA = F32Operand<!TA, BM, THREADS>;
     using OB = F32Operand<TB, BN, THREADS>;
     using OBL = F32Operand<TB, DUAL ? BN / 2 : BN, THREADS>;  // as loaded (DUAL: the gate or up half)
-    static_assert(!DUAL || (!TA && TB), "SwiGLU is Y = X.W^T");
+    static_assert(!DUAL || (!TA && TB && WTN == BN / 2), "SwiGLU is Y = X.W^T, a wave's columns all gate or all up");
     constexpr int SA = OA::STAGE_BYTES;
 
     const int tid = threadIdx.x % THREADS, lane = tid & 63, wave = tid >> 6;
@@ -269,14 +269,17 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
             }
     };
     // Part `part` of `parts` of a register set's split and LDS writes; k0: its k-tile. A k-contiguous
-    // A's elements past K (the next row's) are zeroed; B's then meet zeros, as an mn-contiguous A's
-    // zeros meet them (a B element past K that is not finite costs the wave its second computation).
+    // operand's elements past K (the next row's) are zeroed, in both operands: one that is not finite
+    // would cost the wave its second computation.
     auto gstore = [&](int set, int64_t k0, int part, int parts) {
 #pragma unroll
         for (int q = 0; q < PF; ++q)
             if (q == set) {
-                if constexpr (!TA)
-                    if (part == 0 && k0 + BK > ke) oa[q].mask(ke - k0, tid);
+                if (part == 0 && k0 + BK > ke) {
+                    if constexpr (!TA) oa[q].mask(ke - k0, tid);
+                    if constexpr (TB) ob[q].mask(ke - k0, tid);
+                    if constexpr (DUAL) ob2[q].mask(ke - k0, tid);
+                }
                 oa[q].store(smem, tid, part, parts);
                 ob[q].store(smem + SA, tid, part, parts);
                 if constexpr (DUAL) ob2[q].store(smem + SA + OBL::STAGE_BYTES, tid, part, parts);
@@ -430,34 +433,48 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
         for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j) acc[i][j] = zero;
-        const float *Bw = B;
-        int64_t c0 = n0 + wn * WTN;
-        if constexpr (DUAL) {
-            static_assert(WTN == BN / 2, "a wave's columns are all gate or all up");
-            Bw = wn ? B2 : B;
-            c0 = n0;
-        }
+        // Steps of 16 k: lane group g takes k 4g..4g+3 of both operands, one per MFMA, as the FP32 units'
+        // tiles do; two steps of loads go out together. Elements from ke on are zeros.
+        const bool up = DUAL && __builtin_amdgcn_readfirstlane(wn) != 0;  // this wave's B rows are up-weight rows
+        const int kq = (lane >> 4) * 4;
+        auto quad = [&](const __amdgpu_buffer_rsrc_t &rs, bool kcontig, int64_t ld, int row, int64_t k) {
+            u32x4 v;
+            if (kcontig)
+                v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (uint32_t)((row * ld + k) * 4), 0, 0));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (!kcontig) v[e] = __builtin_amdgcn_raw_buffer_load_b32(rs, (uint32_t)(((k + e) * ld + row) * 4), 0, 0);
+                v[e] = k + e < ke ? v[e] : 0u;
+            }
+            return __builtin_bit_cast(f32x4, v);
+        };
 #pragma unroll 1
-        for (int64_t k0 = kb; k0 < ke; k0 += 4) {
-            const int64_t k = k0 + (lane >> 4);
-            float av[FM], bv[FN];
+        for (int64_t k0 = kb; k0 < ke; k0 += 32) {
+            f32x4 av[2][FM], bv[2][FN];
 #pragma unroll
-            for (int i = 0; i < FM; ++i) {
-                const int64_t row = m0 + wm * WTM + i * 16 + (lane & 15);
-                av[i] = 0.f;
-                if (k < ke && row < p.M) av[i] = A[TA ? k * p.lda + row : row * p.lda + k];
+            for (int h = 0; h < 2; ++h) {
+                const int64_t k = k0 + 16 * h + kq;
+#pragma unroll
+                for (int i = 0; i < FM; ++i) av[h][i] = quad(ra.rs, !TA, p.lda, wm * WTM + i * 16 + (lane & 15), k);
+#pragma unroll
+                for (int j = 0; j < FN; ++j) {
+                    if constexpr (DUAL)
+                        bv[h][j] = up ? quad(rb2.rs, TB, p.ldb, j * 16 + (lane & 15), k)
+                                      : quad(rb.rs, TB, p.ldb, j * 16 + (lane & 15), k);
+                    else
+                        bv[h][j] = quad(rb.rs, TB, p.ldb, wn * WTN + j * 16 + (lane & 15), k);
+                }
             }
 #pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                const int64_t col = c0 + j * 16 + (lane & 15);
-                bv[j] = k < ke && col < p.N ? Bw[TB ? col * p.ldb + k : k * p.ldb + col] : 0.f;
-            }
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int i = 0; i < FM; ++i)
+                for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int j = 0; j < FN; ++j)
-                    acc[i][j] = XPOSE ? __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j], av[i], acc[i][j], 0, 0, 0)
-                                      : __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+                    for (int i = 0; i < FM; ++i)
+#pragma unroll
+                        for (int j = 0; j < FN; ++j)
+                            acc[i][j] = XPOSE ? __builtin_amdgcn_mfma_f32_16x16x4f32(bv[h][j][e], av[h][i][e], acc[i][j], 0, 0, 0)
+                                              : __builtin_amdgcn_mfma_f32_16x16x4f32(av[h][i][e], bv[h][j][e], acc[i][j], 0, 0, 0);
         }
     } else {
 #pragma unroll

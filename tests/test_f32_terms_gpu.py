@@ -146,3 +146,20 @@ def test_small_and_large_operands(it, ta, tb, m, n, k, a_exp, b_exp):
     c = it.gemm(it.Tensor.from_f32_slice(a, a.shape), it.Tensor.from_f32_slice(b, b.shape), trans_a=bool(ta),
                 trans_b=bool(tb))
     _check(c.numpy(), a, b, ta, tb, k)
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", [(300, 260, 520), (1100, 1500, 333), (4100, 2300, 130), (520, 260, 4099)])
+def test_infinities_in_every_wave(it, ta, tb, m, n, k):
+    """An infinity in every 13th row of A (at another k each) sends every wave's tile to the second
+    computation: those rows are the infinities of B's signs, the others finite and within the bound."""
+    a, b = _operands(11, m, n, k, ta, tb)
+    va, vb = op(a, ta), op(b, tb)  # views
+    rows = np.arange(0, m, 13)
+    cols = (rows * 7 + 3) % k
+    va[rows, cols] = np.inf
+    got = it.gemm(it.Tensor.from_f32_slice(a, a.shape), it.Tensor.from_f32_slice(b, b.shape), trans_a=bool(ta),
+                  trans_b=bool(tb)).numpy()
+    assert np.array_equal(got[rows], np.where(vb[cols] > 0, np.inf, -np.inf).astype(np.float32))
+    rest = np.delete(np.arange(m), rows)
+    _check(got[rest], np.ascontiguousarray(va[rest]), np.ascontiguousarray(vb), 0, 0, k)
