@@ -353,30 +353,6 @@ __device__ __forceinline__ void gemm_mfma_block(const GemmArgs &p, int tile, int
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // XF: sums over thousands of tokens, in chunks of 128 k whose results are added with their rounding
-    // errors kept beside them (TwoSum): one chain over 4096 tokens was 2.8e-6 away from the product of the
-    // stored gradient, which the BF16 terms sum to 2e-7.
-    f32x4 total[XF ? FM : 1][XF ? FN : 1], lost[XF ? FM : 1][XF ? FN : 1];
-    if constexpr (XF) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) total[i][j] = lost[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    auto flush = [&]() {
-        if constexpr (XF) {
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j) {
-                    const f32x4 a = total[i][j], b = acc[i][j], s = a + b, bb = s - a;
-                    lost[i][j] += (a - (s - bb)) + (b - bb);
-                    total[i][j] = s;
-                    acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-                }
-        }
-    };
-
     // Register staging sets: PF of them, so the loads of tile t+PF are issued during tile t.
     OA oa[PF];
     constexpr bool RSRC = LM == LOAD_RSRC;
@@ -497,8 +473,6 @@ __device__ __forceinline__ void gemm_mfma_block(const GemmArgs &p, int tile, int
                 }
                 __syncthreads();
                 frags(fa0, fb0, nxt, 0);
-                if constexpr (XF)
-                    if ((t & 3) == 3) flush();
             };
             if constexpr (PF == 1) {
                 for (int t = 0; t < ntiles; ++t) tile(t, 0, 0);
@@ -516,19 +490,6 @@ __device__ __forceinline__ void gemm_mfma_block(const GemmArgs &p, int tile, int
                     if (t + q < ntiles) tile(t + q, q, (q + 1) % PF);
             }
         }
-    }
-
-    if constexpr (XF) {
-        flush();
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float v = total[i][j][e];  // an infinity's rounding error is a NaN
-                    acc[i][j][e] = fabsf(v) < INFINITY ? v + lost[i][j][e] : v;
-                }
     }
 
     // KS: row sums of squares -> 1/rms per block row (the 8 threads of a row are 8 consecutive lanes).

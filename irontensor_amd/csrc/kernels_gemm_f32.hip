@@ -71,8 +71,47 @@ struct F32Operand {
         }
     }
 
+    // Softmax cross-entropy gradient of FP32 logits (the A operand of dL/dh = G.E or dL/dE = G^T.h): the
+    // loaded logits x become (exp(x - max) / sum - onehot) * scale before the split, the exponential
+    // as 2^((x - max) log2 e). Tokens are rows of a k-contiguous tile, whose {max, scale / sum, target}
+    // wait in LDS, and k-rows of an mn-contiguous one, whose statistics come with the tile's loads.
+    struct Xent {
+        const f32x4 *row;  // k-contiguous: per tile row {max, scale / sum, target's bits, -}
+        int64_t c0;        // the tile's first class
+        int left;          // k-contiguous: classes from there on (elements past them are zeros)
+        float scale;
+    };
+    float2 xs[KCONTIG ? 1 : ITERS][LOADS];
+    uint32_t xt[KCONTIG ? 1 : ITERS][LOADS];
+
+    __device__ __forceinline__ void load_xent(const float2 *st, const uint32_t *tg, float scale, int64_t k0,
+                                              int64_t klim, int tid) {
+        static_assert(!KCONTIG, "a k-contiguous tile's tokens are its rows");
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            int kg, rc;
+            unit(tid + it * THREADS, kg, rc);
+#pragma unroll
+            for (int q = 0; q < LOADS; ++q) {
+                const int64_t tok = k0 + kg * KQ + q;
+                const bool ok = tok < klim;  // tokens past the end: zeros
+                const float2 s = st[ok ? tok : klim - 1];
+                const uint32_t t = tg[ok ? tok : klim - 1];
+                xs[it][q] = {ok ? s.x : INFINITY, ok ? s.y * scale : 0.f};
+                xt[it][q] = ok ? t : 0xffffffffu;
+            }
+        }
+    }
+
+    __device__ __forceinline__ static uint32_t xent(uint32_t x, float mx, float ps, bool target, float scale) {
+        constexpr float LOG2E = 1.4426950408889634f;
+        const float g = __builtin_amdgcn_exp2f((__uint_as_float(x) - mx) * LOG2E) * ps - (target ? scale : 0.f);
+        return __float_as_uint(g);
+    }
+
     // Splits and writes part `part` of `parts` of the tile (the caller interleaves them with MFMAs).
-    __device__ __forceinline__ void store(char *lds, int tid, int part, int parts) const {
+    template <bool XF = false>
+    __device__ __forceinline__ void store(char *lds, int tid, int part, int parts, const Xent &x = Xent{}) const {
         constexpr int PIECES = KCONTIG ? ITERS : 4 * ITERS;
         auto mine = [&](int piece) { return piece * parts / PIECES == part; };
 #pragma unroll
@@ -82,7 +121,13 @@ struct F32Operand {
             if constexpr (KCONTIG) {
                 if (!mine(it)) continue;
                 const int rr = item / (BK / VEC), kc = item % (BK / VEC);
-                const u32x4 &v = reg[it][0];
+                u32x4 v = reg[it][0];
+                if constexpr (XF) {
+                    const f32x4 t = x.row[rr];
+                    const int c = kc * VEC, tc = (int)(__float_as_uint(t[2]) - (uint32_t)x.c0);  // target's k in the tile
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = c + e < x.left ? xent(v[e], t[0], t[1], tc == c + e, x.scale) : 0u;
+                }
                 const Bf16x3 a = split_bf16x3(v[0], v[1]), b = split_bf16x3(v[2], v[3]);
                 char *d = lds + off(rr, kc * 8);
 #pragma unroll
@@ -94,9 +139,16 @@ struct F32Operand {
                 for (int j = 0; j < 4; ++j) {
                     if (!mine(it * 4 + j)) continue;
                     char *d = lds + off(rc * 4 + j, kg * KQ * 2);
-                    const Bf16x3 a = split_bf16x3(reg[it][0][j], reg[it][1][j]);
+                    uint32_t v[LOADS];
+#pragma unroll
+                    for (int q = 0; q < LOADS; ++q) {
+                        v[q] = reg[it][q][j];
+                        if constexpr (XF)
+                            v[q] = xent(v[q], xs[it][q].x, xs[it][q].y, xt[it][q] == (uint32_t)(x.c0 + rc * VEC + j), x.scale);
+                    }
+                    const Bf16x3 a = split_bf16x3(v[0], v[1]);
                     if constexpr (KQ == 4) {
-                        const Bf16x3 b = split_bf16x3(reg[it][2][j], reg[it][3][j]);
+                        const Bf16x3 b = split_bf16x3(v[2], v[3]);
 #pragma unroll
                         for (int p = 0; p < 3; ++p) *(u32x2 *)(d + p * PLANE) = u32x2{a.t[p], b.t[p]};
                     } else {
@@ -192,13 +244,15 @@ using S6432 = Shape<64, 32, 2, 2, 2>;    // 32 x 16 per wave, two blocks of eigh
 // FIX (64 x 64 tiles of batch-1 products): with split K, each split's partial tile goes to p.partial
 // at device scope and the tile's last block to arrive at `arrive` (a zero counter, left at zero)
 // adds the splits in split order and runs the epilogue, so no separate reduction launch follows.
-template <class S, bool TA, bool TB, bool DUAL, bool FIX = false>
+// XF: A is the softmax cross-entropy gradient of the logits it holds (F32Operand::Xent).
+template <class S, bool TA, bool TB, bool DUAL, bool FIX = false, bool XF = false>
 __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int64_t z, char *smem0,
                                                int *arrive = nullptr) {
     constexpr int BM = S::BM, BN = S::BN, WM = S::WM, WN = S::WN, KG = S::KG, THREADS = S::THREADS;
     constexpr int BK = ET<float>::BK;
     constexpr int WTM = BM / WM, WTN = BN / WN, FM = WTM / 16, FN = WTN / 16;
-    static_assert(KG == 1 || (BM == 64 && !DUAL && !FIX), "k groups: plain products");
+    static_assert(KG == 1 || (BM == 64 && !DUAL && !FIX && !XF), "k groups: plain products");
+    static_assert(!XF || (!TB && !DUAL && !FIX), "cross-entropy operand: one product, B not transposed");
     // Tiles of 64 rows store straight from transposed accumulators; larger ones stage the epilogue
     // through LDS, whose full-line stores suit outputs of hundreds of megabytes; SwiGLU pairs waves
     // in LDS.
@@ -259,11 +313,21 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
     ra.init(A, p.lda, p.M, p.K, m0, tid);
     rb.init(B, p.ldb, p.N, p.K, n0, tid);
     if constexpr (DUAL) rb2.init(B2, p.ldb, p.N, p.K, n0, tid);
+    __shared__ f32x4 xrow[XF && !TA ? BM : 1];
+    if constexpr (XF && !TA) {
+        for (int r = tid; r < BM; r += THREADS) {
+            const int64_t tok = min(m0 + r, p.M - 1);
+            const float2 st = p.xent_stats[tok];
+            xrow[r] = f32x4{st.x, st.y * p.xent_scale, __uint_as_float(p.xent_tgt[tok]), 0.f};
+        }
+        __syncthreads();
+    }
     auto gload = [&](int set, int64_t k0) {
 #pragma unroll
         for (int q = 0; q < PF; ++q)
             if (q == set) {
                 ra.load(oa[q], k0, tid);
+                if constexpr (XF && TA) oa[q].load_xent(p.xent_stats, p.xent_tgt, p.xent_scale, k0, ke, tid);
                 rb.load(ob[q], k0, tid);
                 if constexpr (DUAL) rb2.load(ob2[q], k0, tid);
             }
@@ -276,11 +340,14 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
         for (int q = 0; q < PF; ++q)
             if (q == set) {
                 if (part == 0 && k0 + BK > ke) {
-                    if constexpr (!TA) oa[q].mask(ke - k0, tid);
+                    if constexpr (!TA && !XF) oa[q].mask(ke - k0, tid);
                     if constexpr (TB) ob[q].mask(ke - k0, tid);
                     if constexpr (DUAL) ob2[q].mask(ke - k0, tid);
                 }
-                oa[q].store(smem, tid, part, parts);
+                if constexpr (XF)
+                    oa[q].template store<true>(smem, tid, part, parts, {xrow, TA ? m0 : k0, (int)min(ke - k0, (int64_t)BK), p.xent_scale});
+                else
+                    oa[q].store(smem, tid, part, parts);
                 ob[q].store(smem + SA, tid, part, parts);
                 if constexpr (DUAL) ob2[q].store(smem + SA + OBL::STAGE_BYTES, tid, part, parts);
             }
@@ -434,7 +501,9 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
 #pragma unroll
             for (int j = 0; j < FN; ++j) acc[i][j] = zero;
         // Steps of 16 k: lane group g takes k 4g..4g+3 of both operands, one per MFMA, as the FP32 units'
-        // tiles do; two steps of loads go out together. Elements from ke on are zeros.
+        // tiles do; two steps of loads go out together (XF: one, for its registers). Elements from ke on
+        // are zeros.
+        constexpr int H = XF ? 1 : 2;
         const bool up = DUAL && __builtin_amdgcn_readfirstlane(wn) != 0;  // this wave's B rows are up-weight rows
         const int kq = (lane >> 4) * 4;
         auto quad = [&](const __amdgpu_buffer_rsrc_t &rs, bool kcontig, int64_t ld, int row, int64_t k) {
@@ -449,13 +518,27 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
             return __builtin_bit_cast(f32x4, v);
         };
 #pragma unroll 1
-        for (int64_t k0 = kb; k0 < ke; k0 += 32) {
-            f32x4 av[2][FM], bv[2][FN];
+        for (int64_t k0 = kb; k0 < ke; k0 += 16 * H) {
+            f32x4 av[H][FM], bv[H][FN];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
+            for (int h = 0; h < H; ++h) {
                 const int64_t k = k0 + 16 * h + kq;
 #pragma unroll
-                for (int i = 0; i < FM; ++i) av[h][i] = quad(ra.rs, !TA, p.lda, wm * WTM + i * 16 + (lane & 15), k);
+                for (int i = 0; i < FM; ++i) {
+                    const int rl = wm * WTM + i * 16 + (lane & 15);
+                    av[h][i] = quad(ra.rs, !TA, p.lda, rl, k);
+                    if constexpr (XF) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int64_t tok = TA ? k + e : m0 + rl, cls = TA ? m0 + rl : k + e;
+                            const bool ok = k + e < ke && m0 + rl < p.M;
+                            const float2 st = ok ? p.xent_stats[tok] : float2{0.f, 0.f};
+                            const bool target = ok && p.xent_tgt[tok] == (uint32_t)cls;
+                            const uint32_t g = OA::xent(__float_as_uint(av[h][i][e]), st.x, st.y * p.xent_scale, target, p.xent_scale);
+                            av[h][i][e] = ok ? __uint_as_float(g) : 0.f;
+                        }
+                    }
+                }
 #pragma unroll
                 for (int j = 0; j < FN; ++j) {
                     if constexpr (DUAL)
@@ -466,7 +549,7 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
                 }
             }
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < H; ++h)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -580,10 +663,10 @@ __device__ __forceinline__ void gemm_f32_block(const GemmArgs &p, int tile, int6
     }
 }
 
-template <class S, bool TA, bool TB, bool DUAL>
+template <class S, bool TA, bool TB, bool DUAL, bool XF = false>
 __global__ __launch_bounds__(S::THREADS * S::KG, S::WAVES) void gemm_f32_terms(const GemmArgs p) {
     __shared__ __attribute__((aligned(16))) char smem[S::KG * S::SMEM];
-    gemm_f32_block<S, TA, TB, DUAL>(p, blockIdx.x, blockIdx.y, smem);
+    gemm_f32_block<S, TA, TB, DUAL, false, XF>(p, blockIdx.x, blockIdx.y, smem);
 }
 
 // A group of GEMMs: 64 x 64 tiles, batch 1, one split count for the group. Split-K partial sums go to
@@ -597,9 +680,9 @@ __global__ __launch_bounds__(S64::THREADS, S64::WAVES) void gemm_f32_terms_group
     gemm_f32_block<S64, TA, TB, false, true>(p, tile, split, smem, grp.arrive + grp.cstart[gi] + tile);
 }
 
-template <class S, bool TA, bool TB, bool DUAL>
+template <class S, bool TA, bool TB, bool DUAL, bool XF = false>
 void go(const GemmArgs &a, dim3 grid, hipStream_t s) {
-    hipLaunchKernelGGL((gemm_f32_terms<S, TA, TB, DUAL>), grid, dim3(S::THREADS * S::KG), 0, s, a);
+    hipLaunchKernelGGL((gemm_f32_terms<S, TA, TB, DUAL, XF>), grid, dim3(S::THREADS * S::KG), 0, s, a);
 }
 
 // bm x bn: the output tile (SwiGLU: half as wide as its B tile).
@@ -646,7 +729,7 @@ Plan choose_plan(const GemmArgs &a, int64_t cus, bool ta, double *est) {
     double best_t = 1e30;
     int64_t best_blocks = 0;
     for (const Tile &tile : {T256, T128, T64, T6432}) {
-        if (tile.bm != tile.bn && !plain) continue;
+        if (tile.bm != tile.bn && (!plain || a.xent_stats)) continue;
         if (tile.bm == 256 && (ta || a.swiglu_bwd || a.rope_table)) continue;
         const int bn = a.dual ? tile.bn / 2 : tile.bn;
         const int64_t tiles = cdiv(a.M, tile.bm) * cdiv(a.N, bn) * a.batch;
@@ -682,7 +765,7 @@ bool f32_terms_applicable(const GemmArgs &a, bool ta, bool tb) {
     // A few rows wait on latency, not on the matrix units: M = 1, N = 768, K = 256 takes 6.7 us here
     // and 6.0 on the FP32 units' 64 x 32 tile, which loads two k-tiles ahead.
     // (X.W^T there goes to gemv_nt where its rows are whole 16-byte chunks.)
-    return a.M > 16 && !a.f32_units && !a.a_kscale && !a.xent_stats && spans_fit(a, ta, tb);
+    return a.M > 16 && !a.f32_units && !a.a_kscale && spans_fit(a, ta, tb);
 }
 
 it_status launch_gemm_f32(it_context *ctx, bool ta, bool tb, GemmArgs a, const char *tag) {
@@ -721,7 +804,7 @@ it_status launch_gemm_f32(it_context *ctx, bool ta, bool tb, GemmArgs a, const c
     if (ctx->profiling) {
         char buf[192];
         std::snprintf(buf, sizeof(buf), "gemm_f32_%c%c_%dx%d%s%s|%s[%lld,%lld,%lld]x%lld s%d", ta ? 'T' : 'N',
-                      tb ? 'T' : 'N', plan.bm, a.dual ? plan.bm : plan.bn, a.dual ? "_swiglu" : "",
+                      tb ? 'T' : 'N', plan.bm, a.dual ? plan.bm : plan.bn, a.dual ? "_swiglu" : a.xent_stats ? "_xent" : "",
                       a.causal || a.kmode ? "_causal" : "", tag ? tag : "", (long long)a.M, (long long)a.N,
                       (long long)a.K, (long long)a.batch, a.splits);
         key = buf;
@@ -731,6 +814,9 @@ it_status launch_gemm_f32(it_context *ctx, bool ta, bool tb, GemmArgs a, const c
     if (a.dual) {  // X.W^T (checked by the caller)
         if (plan.bm == 128) go<S128, false, true, true>(a, grid, s);
         else go<S64, false, true, true>(a, grid, s);
+    } else if (a.xent_stats) {  // B not transposed (checked by the caller)
+        if (plan.bm == 128) ta ? go<S128, true, false, false, true>(a, grid, s) : go<S128, false, false, false, true>(a, grid, s);
+        else ta ? go<S64, true, false, false, true>(a, grid, s) : go<S64, false, false, false, true>(a, grid, s);
     } else if (!ta && !tb) {
         launch_plain<false, false>(plan.bm, plan.bn, a, grid, s);
     } else if (!ta && tb) {
@@ -760,8 +846,8 @@ bool launch_gemm_f32_group(it_context *ctx, bool ta, bool tb, const GemmArgs *ar
     double separate = 0.0;
     for (int i = 0; i < count; ++i) {
         const GemmArgs &a = args[i];
-        if (a.batch != 1 || a.dual || a.causal != CAUSAL_NONE || a.kmode != KMODE_FULL || a.swiglu_bwd || a.K <= 0 ||
-            a.N % 4 != 0 || a.no_split)
+        if (a.batch != 1 || a.dual || a.causal != CAUSAL_NONE || a.kmode != KMODE_FULL || a.swiglu_bwd || a.xent_stats ||
+            a.K <= 0 || a.N % 4 != 0 || a.no_split)
             return false;
         double t = 0.0;
         choose_plan(a, cus, ta, &t);

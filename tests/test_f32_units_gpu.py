@@ -52,3 +52,41 @@ def test_swiglu_weights_inside_nan(it, rows, h, f):
     gate, up = g[1:-1].astype(np.float64), u[1:-1].astype(np.float64)
     ref = gate / (1 + np.exp(-gate)) * up
     assert np.max(np.abs(hh[1:-1] - ref)) <= 4e-6 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("units", [False, True])
+@pytest.mark.parametrize("tokens,vocab,h", [(4096, 16384, 256), (129, 1001, 65), (70, 34, 33), (333, 5003, 300)])
+def test_cross_entropy_operand(it, units, tokens, vocab, h):
+    """dh = G.E and dE = G^T.h with G = (softmax - onehot) / T rebuilt from the logits, on the terms and on the
+    FP32 units, against float64; an infinity in the other operand reaches its own column alone (the
+    terms' second computation rebuilds G as well)."""
+    from irontensor_amd import train_ops
+    logits = synth.normal(1, (tokens, vocab), std=3.0)
+    hid, emb = synth.normal(2, (tokens, h)), synth.normal(3, (vocab, h), std=0.02)
+    tg = synth.tokens(4, tokens, vocab)
+    hid[min(40, tokens - 1), h - 1] = np.inf
+    emb[min(40, vocab - 1), 0] = np.inf
+    T = it.Tensor.from_f32_slice
+    L, Hd, E = T(logits, logits.shape), T(hid, hid.shape), T(emb, emb.shape)
+    _, _, stats = train_ops.cross_entropy_stats(L, tg)
+    ids = train_ops.upload_ids(tg, vocab)
+    epi = _lib.Epilogue(flags=_lib.IT_EPI_XENT_A | (_lib.IT_EPI_F32_UNITS if units else 0), xent_stats=stats.ptr,
+                        xent_targets=ids.ptr, xent_scale=1.0 / tokens)
+    dh, de = it.Tensor.empty([tokens, h]), it.Tensor.empty([vocab, h])
+    ctx = L.ctx
+    for ta, a, b, c, m, k in ((0, L, E, dh, tokens, vocab), (1, L, Hd, de, vocab, tokens)):
+        st = ctx.lib.it_gemm(ctx.handle, 0, 0, ta, 0, m, h, k, 1.0, C.c_void_p(a.ptr), vocab, 0, C.c_void_p(b.ptr), h,
+                             0, 0.0, C.c_void_p(c.ptr), h, 0, 1, C.byref(epi))
+        assert st == 0
+    x = logits.astype(np.float64)
+    p = np.exp(x - x.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    p[np.arange(tokens), tg] -= 1.0
+    p /= tokens
+    # The sums' bound, and the rebuilt element's own: exp2 of a rounded argument, about 1e-6 of it.
+    for got, A, B, bad in ((dh.numpy(), p, emb, 0), (de.numpy(), p.T, hid, h - 1)):
+        assert not np.isfinite(got[:, bad]).any()
+        fine = np.arange(h) != bad
+        A, B = np.ascontiguousarray(A), B[:, fine].astype(np.float64)
+        n = A.shape[1]
+        assert np.all(np.abs(got[:, fine] - A @ B) <= ((n + 2) * 2.0 ** -24 + 3e-6) * (np.abs(A) @ np.abs(B)))
