@@ -696,16 +696,20 @@ void launch_plain(int bm, int bn, const GemmArgs &a, dim3 grid, hipStream_t s) {
 }
 
 // The tiles as the planner prices them, in microseconds: a k-tile of a block that shares its CU (its
-// share of the CU's time) and of one that has it alone, and a round's prologue and epilogue, fitted on
-// timings of every tile and split on the TINY step's shapes, ragged ones and 4096^3.
+// share of the CU's time) and of one that has it alone, a round's launch, prologue and epilogue, and what a
+// transposed A costs a k-tile (64-byte pieces of its rows, which the 64 x 32 tile waits for). Fitted on
+// every tile and split count of 110 shapes, warm: the TINY step's, ragged ones, squares, and random ones
+// of 17 to 8192 rows and up to 16384 columns and 11008 k. The picks take 1.3% longer than the fastest
+// measured plans; the former constants, with powers of two as split counts, took 5.4%, up to 1.4x
+// ([701, 300, 1000] of a transposed A 19.7 us on 64 x 32 tiles, 14.8 on 64 x 64 with four splits).
 struct Tile {
     int bm, bn, occ;  // occ: blocks a CU runs at once
-    double shared, alone, round;
+    double shared, alone, round, ta;
 };
-// 256 x 128 before 128 x 128, which it beats by 3% where both fill the GPU (4096^3 651 against 674 us,
-// [4096, 256, 16384] 197 against 203).
-constexpr Tile T256{256, 128, 1, 2.55, 2.55, 8.0}, T128{128, 128, 2, 1.31, 1.75, 4.5},
-    T64{64, 64, 3, 0.45, 0.60, 3.0}, T6432{64, 32, 2, 0.268, 0.30, 3.0};
+constexpr Tile T256{256, 128, 1, 2.08, 2.43, 15.4, 1.0}, T128{128, 128, 2, 1.36, 2.41, 12.6, 1.0},
+    T64{64, 64, 3, 0.52, 0.69, 4.8, 1.0}, T6432{64, 32, 2, 0.307, 0.34, 4.9, 1.5};
+constexpr double PARTIAL_BW = 3.1e12, REDUCE = 1.6e-6;  // split-K partial sums out and back, the reduction
+constexpr int SPLITS[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
 
 struct Plan {
     int bm, bn, splits;
@@ -713,12 +717,23 @@ struct Plan {
 };
 
 // One launch of `blocks` blocks of ksteps k-tiles, in seconds.
-double launch_time(const Tile &t, int64_t blocks, int64_t ksteps, int64_t cus) {
+double launch_time(const Tile &t, bool ta, int64_t blocks, int64_t ksteps, int64_t cus) {
     const int64_t per_cu = cdiv(blocks, cus), conc = std::min<int64_t>(per_cu, t.occ);
-    return 1e-6 * cdiv(per_cu, t.occ) * (t.round + ksteps * std::max(conc * t.shared, t.alone));
+    return 1e-6 * cdiv(per_cu, t.occ) * (t.round + (ta ? t.ta : 1.0) * ksteps * std::max(conc * t.shared, t.alone));
 }
 
-// Picks the tile and a power-of-two split count, lowest price first. Near ties (3%) keep the earlier
+// A group's launch of 64 x 64 blocks, in seconds: its rounds overlap less evenly than one product's, so a
+// last round that a few blocks fill costs what they take alone. Fitted on eleven groups of two to four
+// products: the split counts it picks take 0.1% longer than the fastest (the TINY layer's four weight
+// gradients: five splits, 980 blocks, 65.5 us; four, 784 blocks in one round and 16 more, 75.6).
+double group_time(int64_t blocks, int64_t ksteps, int64_t cus) {
+    constexpr Tile t{64, 64, 3, 0.50, 0.60, 3.0, 1.0};
+    const int64_t full = blocks / (t.occ * cus), rest = cdiv(blocks % (t.occ * cus), cus);
+    return 1e-6 * (full * (t.round + ksteps * std::max(t.occ * t.shared, t.alone)) +
+                   (rest ? t.round + ksteps * std::max(rest * t.shared, t.alone) : 0.0));
+}
+
+// Picks the tile and the split count, lowest price first. Near ties (3%) keep the earlier
 // plan, except that between two unsplit plans the one with more blocks wins (more loads in flight per
 // k-step); the 64 x 32 tile has to win outright.
 Plan choose_plan(const GemmArgs &a, int64_t cus, bool ta, double *est) {
@@ -733,13 +748,13 @@ Plan choose_plan(const GemmArgs &a, int64_t cus, bool ta, double *est) {
         if (tile.bm == 256 && (ta || a.swiglu_bwd || a.rope_table)) continue;
         const int bn = a.dual ? tile.bn / 2 : tile.bn;
         const int64_t tiles = cdiv(a.M, tile.bm) * cdiv(a.N, bn) * a.batch;
-        for (int s = 1; s <= 32; s *= 2) {
+        for (const int s : SPLITS) {
             if (s > 1 && (!plain || a.no_split)) break;
             const int64_t kps = s == 1 ? kall : cdiv(cdiv(a.K, s), bk) * bk;
             if (s > 1 && kps < 4 * bk) break;
             const int64_t splits = s > 1 ? cdiv(a.K, kps) : 1, blocks = tiles * splits;
-            double t = launch_time(tile, blocks, kps / bk, cus);
-            if (splits > 1) t += 2.0 * splits * a.M * a.N * a.batch * 4.0 / 4e12 + 4e-6;  // partial sums, reduction
+            double t = launch_time(tile, ta, blocks, kps / bk, cus);
+            if (splits > 1) t += 2.0 * splits * a.M * a.N * a.batch * 4.0 / PARTIAL_BW + REDUCE;
             const bool better = t < best_t * 0.97;
             const bool tie_more_blocks = t < best_t * 1.03 && splits == 1 && best.splits == 1 &&
                                          blocks > best_blocks && tile.bn != 32;
@@ -765,6 +780,11 @@ bool f32_terms_applicable(const GemmArgs &a, bool ta, bool tb) {
     // A few rows wait on latency, not on the matrix units: M = 1, N = 768, K = 256 takes 6.7 us here
     // and 6.0 on the FP32 units' 64 x 32 tile, which loads two k-tiles ahead.
     // (X.W^T there goes to gemv_nt where its rows are whole 16-byte chunks.)
+    // More rows stay here for their precision also where the FP32 units are faster, which they are in
+    // products of few k-tiles (a k-tile's split sits between its load and its products): K = 256 FP32
+    // units 2.9e-7 from 64 bits and 9.9 us against 0.9e-7 and 11.6 ([4096, 256, 256], X.W), 512^3 9.6
+    // against 11.9. Over 110 shapes (choose_plan) the terms are 1.10x as fast, from 0.66x ([192, 176, 160] of
+    // a transposed A) to 2.1x; callers that would rather have the time ask for the units (IT_EPI_F32_UNITS).
     return a.M > 16 && !a.f32_units && !a.a_kscale && spans_fit(a, ta, tb);
 }
 
@@ -872,8 +892,8 @@ bool launch_gemm_f32_group(it_context *ctx, bool ta, bool tb, const GemmArgs *ar
             if (splits > 1) traffic += 2.0 * splits * a.M * a.N * 4.0;
         }
         if (!ok) break;
-        double t = launch_time(T64, blocks, ksteps, cus);
-        if (traffic > 0.0) t += traffic / 4e12 + 4e-6;  // partial sums out and back, the tiles' last-block sums
+        double t = group_time(blocks, ksteps, cus);
+        if (traffic > 0.0) t += traffic / PARTIAL_BW + REDUCE;  // the tiles' last blocks add the partial sums
         if (t < best_t) {
             best_t = t;
             best_s = s;
