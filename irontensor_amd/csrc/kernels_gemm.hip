@@ -1811,11 +1811,6 @@ bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &p
     return best + copies < t_plain && r.bytes_a + r.bytes_b <= (size_t(1) << 30);
 }
 
-// Whether the scratch can be had now: a capture may not allocate.
-bool scratch_ready(const it_context *ctx, size_t bytes) {
-    return !ctx->capturing || ctx->scratch_bytes[ctx->cur] >= bytes;
-}
-
 it_status launch_ragged(it_context *ctx, bool ta, bool tb, GemmArgs a, const Ragged &r, void *ws, const char *tag) {
     std::string key;
     hipEvent_t ev = nullptr;
@@ -1941,9 +1936,11 @@ it_status launch_gemm(it_context *ctx, it_dtype dtype_in, bool transA, bool tran
     if (Ragged r; bf16 && plan_ragged(a, cus, transA, transB, plan, t_plan, r)) {
         const size_t bytes = r.bytes_a + r.bytes_b + r.bytes_part;
         void *ws = nullptr;
-        if (a.batch * r.plan.splits <= 65535 && scratch_ready(ctx, bytes) &&
-            (bytes == 0 || ensure_scratch(ctx, bytes, &ws) == IT_OK))
-            return launch_ragged(ctx, transA, transB, a, r, ws, profile_tag);
+        if (a.batch * r.plan.splits <= 65535) {
+            if (bytes == 0 || ensure_scratch(ctx, bytes, &ws) == IT_OK)
+                return launch_ragged(ctx, transA, transB, a, r, ws, profile_tag);
+            clear_error();  // no scratch (a capture may not allocate): the plain tiles
+        }
     }
 #ifdef IT_TUNING
     // Planner sweeps only (a tuning build): IT_PLAN="tile,splits[,width]" forces the plan.

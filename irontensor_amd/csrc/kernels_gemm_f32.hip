@@ -790,11 +790,6 @@ bool f32_terms_applicable(const GemmArgs &a, bool ta, bool tb) {
 
 it_status launch_gemm_f32(it_context *ctx, bool ta, bool tb, GemmArgs a, const char *tag) {
     Plan plan = choose_plan(a, cus_of(ctx), ta, nullptr);
-    if (plan.splits > 1 && ctx->capturing &&
-        ctx->scratch_bytes[ctx->cur] < (size_t)plan.splits * a.batch * a.M * a.N * sizeof(float)) {
-        a.no_split = 1;  // a capture may not allocate
-        plan = choose_plan(a, cus_of(ctx), ta, nullptr);
-    }
 #ifdef IT_TUNING
     // Planner sweeps only (a tuning build): IT_PLAN="tile,splits[,width]" forces the plan.
     if (const char *env = std::getenv("IT_PLAN")) {
@@ -803,15 +798,22 @@ it_status launch_gemm_f32(it_context *ctx, bool ta, bool tb, GemmArgs a, const c
         if (n >= 2) plan = Plan{bm, a.dual ? bm / 2 : n == 3 ? bn : bm, sp, cdiv(cdiv(a.K, sp), 32) * 32};
     }
 #endif
-    a.tiles_m = (int)cdiv(a.M, plan.bm);
-    a.tiles_n = (int)cdiv(a.N, plan.bn);
-    a.k_per_split = plan.k_per_split;
-    a.splits = (int)std::max<int64_t>(1, cdiv(a.K, plan.k_per_split));
+    auto apply = [&](const Plan &pl) {
+        plan = pl;
+        a.tiles_m = (int)cdiv(a.M, pl.bm);
+        a.tiles_n = (int)cdiv(a.N, pl.bn);
+        a.k_per_split = pl.k_per_split;
+        a.splits = (int)std::max<int64_t>(1, cdiv(a.K, pl.k_per_split));
+    };
+    apply(plan);
     any_alignment(a);
     if (a.splits > 1) {
         void *ws = nullptr;
-        const it_status st = ensure_scratch(ctx, (size_t)a.splits * a.batch * a.M * a.N * sizeof(float), &ws);
-        if (st != IT_OK) return st;
+        if (ensure_scratch(ctx, (size_t)a.splits * a.batch * a.M * a.N * sizeof(float), &ws) != IT_OK) {
+            clear_error();
+            a.no_split = 1;  // no scratch (a capture may not allocate): the best plan without
+            apply(choose_plan(a, cus_of(ctx), ta, nullptr));
+        }
         a.partial = (float *)ws;
     }
     const int64_t gx = (int64_t)a.tiles_m * a.tiles_n, gy = a.batch * a.splits;
@@ -934,14 +936,12 @@ bool launch_gemm_f32_group(it_context *ctx, bool ta, bool tb, const GemmArgs *ar
     const int grid_blocks = xcd_schedule(grp);
     if (!grid_blocks) return false;
     if (split_any) {
-        if (ctx->capturing &&
-            (!ctx->counters[ctx->cur] || ctx->scratch_bytes[ctx->cur] < (size_t)scratch * sizeof(float)))
-            return false;  // a capture may not allocate
-        *status = ensure_counters(ctx, &grp.arrive);
-        if (*status != IT_OK) return true;
         void *ws = nullptr;
-        *status = ensure_scratch(ctx, (size_t)scratch * sizeof(float), &ws);
-        if (*status != IT_OK) return true;
+        if (ensure_counters(ctx, &grp.arrive) != IT_OK ||
+            ensure_scratch(ctx, (size_t)scratch * sizeof(float), &ws) != IT_OK) {
+            clear_error();
+            return false;  // no scratch (a capture may not allocate): separate products
+        }
         float *part = (float *)ws;
         for (int i = 0; i < count; ++i)
             if (grp.g[i].splits > 1) {

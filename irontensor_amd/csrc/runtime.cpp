@@ -44,6 +44,17 @@ it_status join_side(it_context *ctx) {
     return IT_OK;
 }
 
+// hipMalloc whose failure leaves no error pending: the caller may go on without the block, and its next
+// launch must not report it.
+static hipError_t device_alloc(void **p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
 static it_status grow(it_context *ctx, void *&buf, size_t &have, size_t bytes, void **out) {
     if (have < bytes && ctx->capturing)
         return fail(IT_ERR_INVALID, "scratch of " + std::to_string(bytes) +
@@ -62,7 +73,7 @@ static it_status grow(it_context *ctx, void *&buf, size_t &have, size_t bytes, v
             have = 0;
         }
         size_t want = bytes < (size_t(64) << 20) ? (size_t(64) << 20) : bytes;
-        IT_HIP_TRY(hipMalloc(&buf, want));
+        IT_HIP_TRY(device_alloc(&buf, want));
         have = want;
     }
     *out = buf;
@@ -82,7 +93,7 @@ it_status ensure_counters(it_context *ctx, int **out) {
     if (!f) {
         if (ctx->capturing)
             return fail(IT_ERR_INVALID, "arrival counters needed during graph capture: run the work once before capturing");
-        IT_HIP_TRY(hipMalloc(&f, COUNTERS * sizeof(int)));
+        IT_HIP_TRY(device_alloc((void **)&f, COUNTERS * sizeof(int)));
         // Synchronous zero fill at allocation (never inside a captured graph).
         hipError_t e = hipMemset(f, 0, COUNTERS * sizeof(int));
         if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -257,14 +268,13 @@ it_status it_malloc(it_context *ctx, size_t bytes, void **out_ptr) {
         if (ctx->capturing)
             return fail(IT_ERR_INVALID, "it_malloc: no cached block of " + std::to_string(sz) +
                                             " bytes during graph capture");
-        hipError_t e = hipMalloc(&p, sz);
+        hipError_t e = it::device_alloc(&p, sz);
         if (e != hipSuccess) {
             // Release the cache once and retry before giving up.
             (void)it::sync_all(ctx);
             for (auto &kv : ctx->cache) (void)hipFree(kv.second);
             ctx->cache.clear();
-            (void)hipGetLastError();
-            e = hipMalloc(&p, sz);
+            e = it::device_alloc(&p, sz);
             if (e != hipSuccess)
                 return fail(IT_ERR_OOM, "it_malloc: failed to allocate " + std::to_string(sz) +
                                             " bytes: " + hipGetErrorString(e));
