@@ -1709,6 +1709,7 @@ struct PadSide {
     int64_t s_in, s_out, ld;
     uint16_t *dst;
     uint32_t rows, cols, rows_p, vecs;  // vecs = dst_ld / 8
+    uint32_t items;                     // batch items to copy: one for an operand that all of them share
 };
 struct PadArgs {
     PadSide side[2];
@@ -1721,6 +1722,7 @@ struct PadArgs {
 __global__ __launch_bounds__(256) void pad_bf16(const PadArgs p) {
     const PadSide o = p.side[blockIdx.z];
     const int64_t b = blockIdx.y;
+    if (b >= o.items) return;
     const uint16_t *src = o.src + b / p.inner * o.s_out + b % p.inner * o.s_in;
     uint16_t *dst = o.dst + b * o.rows_p * o.vecs * 8;
     const uint32_t total = o.rows_p * o.vecs;  // the copies take at most 1 GB
@@ -1747,6 +1749,7 @@ __global__ __launch_bounds__(256) void pad_bf16(const PadArgs p) {
 struct Ragged {
     Plan plan;
     bool copy_a, copy_b;
+    int64_t items_a, items_b;                // batch items of the copies
     int64_t kp, rows_a, ld_a, rows_b, ld_b;  // K padded; the copies' shapes (stored layout)
     size_t bytes_a, bytes_b, bytes_part;     // scratch: the copies and the split-K partial sums
 };
@@ -1778,8 +1781,10 @@ bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &p
     r.ld_a = ta ? cdiv(a.M, 8) * 8 : r.kp;
     r.rows_b = tb ? a.N : r.kp;
     r.ld_b = tb ? r.kp : cdiv(a.N, 8) * 8;
-    r.bytes_a = r.copy_a ? align256((size_t)a.batch * r.rows_a * r.ld_a * 2) : 0;
-    r.bytes_b = r.copy_b ? align256((size_t)a.batch * r.rows_b * r.ld_b * 2) : 0;
+    r.items_a = a.sA_in == 0 && a.sA_out == 0 ? 1 : a.batch;
+    r.items_b = a.sB_in == 0 && a.sB_out == 0 ? 1 : a.batch;
+    r.bytes_a = r.copy_a ? align256((size_t)r.items_a * r.rows_a * r.ld_a * 2) : 0;
+    r.bytes_b = r.copy_b ? align256((size_t)r.items_b * r.rows_b * r.ld_b * 2) : 0;
     const double copies = ((r.copy_a || r.copy_b) ? 3e-6 : 0.0) + 2.0 * (r.bytes_a + r.bytes_b) / 2.5e12;
     double best = 1e30;
     for (const int unit : {256, 128}) {  // whole tiles of this unit cover the product
@@ -1825,25 +1830,26 @@ it_status launch_ragged(it_context *ctx, bool ta, bool tb, GemmArgs a, const Rag
     PadArgs pad{};
     pad.inner = a.batch_inner;
     int sides = 0;
-    int64_t most = 0;  // 16-byte vectors of the larger copy
+    int64_t most = 0, items_most = 1;  // 16-byte vectors of the larger copy, items of the more numerous
     char *at = (char *)ws;
     auto copy = [&](const void *&src, int64_t &s_in, int64_t &s_out, int64_t &ld, int64_t rows, int64_t cols,
-                    int64_t rows_p, int64_t dst_ld, size_t bytes) {
+                    int64_t rows_p, int64_t dst_ld, int64_t items, size_t bytes) {
         pad.side[sides++] = PadSide{(const uint16_t *)src, s_in, s_out, ld, (uint16_t *)at, (uint32_t)rows,
-                                    (uint32_t)cols, (uint32_t)rows_p, (uint32_t)(dst_ld / 8)};
+                                    (uint32_t)cols, (uint32_t)rows_p, (uint32_t)(dst_ld / 8), (uint32_t)items};
         most = std::max(most, rows_p * (dst_ld / 8));
         src = at;
         ld = dst_ld;
-        s_in = rows_p * dst_ld;
+        s_in = items == 1 ? 0 : rows_p * dst_ld;
         s_out = a.batch_inner * s_in;
+        items_most = std::max(items_most, items);
         at += bytes;
     };
     if (r.copy_a)
-        copy(a.A, a.sA_in, a.sA_out, a.lda, ta ? a.K : a.M, ta ? a.M : a.K, r.rows_a, r.ld_a, r.bytes_a);
+        copy(a.A, a.sA_in, a.sA_out, a.lda, ta ? a.K : a.M, ta ? a.M : a.K, r.rows_a, r.ld_a, r.items_a, r.bytes_a);
     if (r.copy_b)
-        copy(a.B, a.sB_in, a.sB_out, a.ldb, tb ? a.N : a.K, tb ? a.K : a.N, r.rows_b, r.ld_b, r.bytes_b);
+        copy(a.B, a.sB_in, a.sB_out, a.ldb, tb ? a.N : a.K, tb ? a.K : a.N, r.rows_b, r.ld_b, r.items_b, r.bytes_b);
     if (sides) {
-        const dim3 grid((unsigned)std::min<int64_t>(cdiv(most, 256), 8192), (unsigned)a.batch, (unsigned)sides);
+        const dim3 grid((unsigned)std::min<int64_t>(cdiv(most, 256), 8192), (unsigned)items_most, (unsigned)sides);
         hipLaunchKernelGGL(pad_bf16, grid, dim3(256), 0, ctx->stream, pad);
     }
     a.partial = (float *)at;

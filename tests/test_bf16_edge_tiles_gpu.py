@@ -8,7 +8,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from irontensor_amd import profiler, synth
+from irontensor_amd import _lib, profiler, synth
 from tests.numerics import op
 
 pytestmark = pytest.mark.gpu
@@ -102,3 +102,41 @@ def test_capture_without_scratch_takes_the_plain_tiles(it):
         assert ctx.lib.it_graph_launch(ctx.handle, g) == 0
         assert np.array_equal(out.numpy(), ref)
     assert ctx.lib.it_graph_destroy(g) == 0
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_batched_epilogues_on_edge_tiles(it, ta, tb, shared):
+    """A batch on padded copies and edge tiles, B its own or shared by the items: alpha, beta and a bias
+    into FP32 and BF16 outputs of odd rows (8-byte stores at 2-byte alignment)."""
+    bt, m, n, k = 3, 700, 901, 333
+    a = synth.small_ints(21, (bt, k, m) if ta else (bt, m, k), -2, 2)
+    b = synth.small_ints(22, ((1,) if shared else (bt,)) + ((n, k) if tb else (k, n)), -2, 2)
+    bias, c0 = synth.small_ints(23, (n,), -4, 4), synth.small_ints(24, (bt, m, n), -4, 4)
+    A, B, Bias = _bf16(it, a), _bf16(it, b), it.Tensor.from_f32_slice(bias, [n])
+    ctx = it.Context.global_()
+    exact = 2 * (np.matmul(op(a, ta).astype(np.float64), op(b, tb).astype(np.float64))) + bias
+    for bf16 in (False, True):
+        beta = 0.0 if bf16 else 3.0
+        out = _bf16(it, c0) if bf16 else it.Tensor.from_f32_slice(c0, list(c0.shape))
+        epi = _lib.Epilogue(flags=_lib.IT_EPI_BIAS, bias=Bias.ptr)
+        keys = _keys(it, lambda: ctx.lib.it_gemm(
+            ctx.handle, 2, 2 if bf16 else 0, ta, tb, m, n, k, 2.0, C.c_void_p(A.ptr), m if ta else k, m * k,
+            C.c_void_p(B.ptr), k if tb else n, 0 if shared else n * k, beta, C.c_void_p(out.ptr), n, m * n, bt, C.byref(epi)))
+        assert len(keys) == 1 and "_dtl_edge|" in keys[0], keys
+        want = (exact + beta * c0).astype(np.float32)
+        got = out.as_bf16_slice().reshape(want.shape) if bf16 else out.numpy()
+        assert np.array_equal(got, it.f32_to_bf16(want) if bf16 else want)
+
+
+@pytest.mark.parametrize("ta,tb,m,n,k", [(0, 0, 246, 656, 9110), (1, 1, 529, 210, 6306), (0, 1, 995, 2294, 4345),
+                                         (1, 0, 991, 1358, 10784)])
+def test_split_k_on_edge_tiles(it, ta, tb, m, n, k):
+    """Few tiles and a long ragged k: the edge tiles' partial sums and their reduction."""
+    a = synth.small_ints(31, (k, m) if ta else (m, k), -2, 2)
+    b = synth.small_ints(32, (n, k) if tb else (k, n), -2, 2)
+    out = it.Tensor.empty([m, n], it.Precision.FP32)
+    keys = _keys(it, lambda: it.gemm(_bf16(it, a), _bf16(it, b), trans_a=bool(ta), trans_b=bool(tb), out=out))
+    print(f"[bf16 edge split] {keys}", flush=True)
+    assert "_dtl_edge|" in keys[0] and not keys[0].endswith(" s1"), keys
+    assert np.array_equal(out.numpy(), (op(a, ta).astype(np.float64) @ op(b, tb).astype(np.float64)).astype(np.float32))

@@ -80,3 +80,15 @@ for f, needs in ((ragged, '_dtl_edge'), (split, ' s'), (group, '_group')):
     assert any(needs in k for k in got), got
 assert not keys(split)[0].endswith(' s1')
 """)
+
+
+def test_shared_operand_is_padded_once(fake):
+    """A ragged BF16 B that a batch shares (stride 0) takes one padded copy: forty of this one would pass the
+    1 GB that such copies may take, and the product would stay on the plain tiles."""
+    _run(fake, """
+bt, m, n, k = 40, 128, 4097, 4001
+A, B, Cc = buf(bt * m * k // 2 + 1), buf(n * k // 2 + 1), buf(bt * m * n)
+got = keys(lambda: gemm(1, 0, 1, m, n, k, A.ptr, B.ptr, Cc.ptr, bt, m * k, 0, m * n))
+print(got)
+assert '_dtl_edge' in got[0], got
+""")
