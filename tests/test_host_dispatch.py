@@ -92,3 +92,14 @@ got = keys(lambda: gemm(1, 0, 1, m, n, k, A.ptr, B.ptr, Cc.ptr, bt, m * k, 0, m 
 print(got)
 assert '_dtl_edge' in got[0], got
 """)
+
+
+def test_ragged_products_run_the_plan_that_was_priced(fake):
+    """A long ragged k whose plain plan is 256 x 256 tiles with split K: the edge tiles take the plan their
+    price is for, here one round of 256 x 128 tiles."""
+    _run(fake, """
+X = buf(1 << 25)
+got = keys(lambda: gemm(1, 1, 0, 1928, 2872, 1936, X.ptr, X.ptr, X.ptr))
+print(got)
+assert '_256x128_dtl_edge|' in got[0] and got[0].endswith(' s1'), got
+""")
