@@ -1811,6 +1811,7 @@ bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &p
             r.plan = pl;
         }
     }
+    if (best >= 1e30) return false;  // no direct-to-LDS tile spans the operands in place
     r.bytes_part = r.plan.splits > 1 ? (size_t)r.plan.splits * a.batch * a.M * a.N * sizeof(float) : 0;
     return best + copies < t_plain && r.bytes_a + r.bytes_b <= (size_t(1) << 30);
 }

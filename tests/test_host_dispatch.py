@@ -103,3 +103,14 @@ got = keys(lambda: gemm(1, 1, 0, 1928, 2872, 1936, X.ptr, X.ptr, X.ptr))
 print(got)
 assert '_256x128_dtl_edge|' in got[0] and got[0].endswith(' s1'), got
 """)
+
+
+def test_operands_beyond_the_edge_tiles_offsets(fake):
+    """A ragged product over a B whose k rows span more than 2 GiB a split has no edge-tile plan and stays on
+    the plain tiles (launched on nothing here: the buffer is not that large)."""
+    _run(fake, """
+X = buf(1 << 22)
+got = keys(lambda: gemm(1, 0, 0, 1000, 1000, 4096, X.ptr, X.ptr, X.ptr, ldb=1 << 23))
+print(got)
+assert '_edge' not in got[0], got
+""")
