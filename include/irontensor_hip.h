@@ -77,7 +77,8 @@ size_t it_mem_allocated(it_context *ctx);
  * retired while graphs that may use them are alive (see it_graph_launch). The reference allocates
  * per op and has no such pool. */
 size_t it_mem_scratch(it_context *ctx);
-/* Returns cached blocks to the device. */
+/* Returns cached blocks to the device, and the scratch of padded operand copies (ragged BF16 products, up
+ * to 1 GB) unless a graph captured on this context is alive. */
 it_status it_empty_cache(it_context *ctx);
 
 /* Copies. h2d and d2d are stream-ordered; d2h blocks until the data is on the host (the reference's

@@ -66,6 +66,9 @@ struct it_context {
     size_t scratch_bytes[2] = {0, 0};
     void *attn_scratch[2] = {nullptr, nullptr};
     size_t attn_scratch_bytes[2] = {0, 0};
+    // Padded operand copies (ragged BF16 products; up to 1 GB), given back by it_empty_cache.
+    void *pad_scratch[2] = {nullptr, nullptr};
+    size_t pad_scratch_bytes[2] = {0, 0};
     // Scratch blocks replaced by a larger one while graphs captured on this context were alive: a
     // graph keeps the addresses it was captured with, so the old block stays allocated until the
     // last such graph is destroyed (or the context shuts down).
@@ -109,6 +112,7 @@ it_status join_side(it_context *ctx);
 // Grows the current stream's scratch to at least `bytes` (synchronises before freeing the old block).
 it_status ensure_scratch(it_context *ctx, size_t bytes, void **out);
 it_status ensure_attn_scratch(it_context *ctx, size_t bytes, void **out);
+it_status ensure_pad_scratch(it_context *ctx, size_t bytes, void **out);
 // The current stream's arrival counters (COUNTERS ints, zero), allocated on first use.
 constexpr int64_t COUNTERS = 1 << 16;
 it_status ensure_counters(it_context *ctx, int **out);

@@ -1751,7 +1751,7 @@ struct Ragged {
     bool copy_a, copy_b;
     int64_t items_a, items_b;                // batch items of the copies
     int64_t kp, rows_a, ld_a, rows_b, ld_b;  // K padded; the copies' shapes (stored layout)
-    size_t bytes_a, bytes_b, bytes_part;     // scratch: the copies and the split-K partial sums
+    size_t bytes_a, bytes_b, bytes_part;     // the copies' scratch and that of the split-K partial sums
 };
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
@@ -1816,7 +1816,8 @@ bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &p
     return best + copies < t_plain && r.bytes_a + r.bytes_b <= (size_t(1) << 30);
 }
 
-it_status launch_ragged(it_context *ctx, bool ta, bool tb, GemmArgs a, const Ragged &r, void *ws, const char *tag) {
+it_status launch_ragged(it_context *ctx, bool ta, bool tb, GemmArgs a, const Ragged &r, void *pads, void *part,
+                        const char *tag) {
     std::string key;
     hipEvent_t ev = nullptr;
     if (ctx->profiling) {
@@ -1831,7 +1832,7 @@ it_status launch_ragged(it_context *ctx, bool ta, bool tb, GemmArgs a, const Rag
     pad.inner = a.batch_inner;
     int sides = 0;
     int64_t most = 0, items_most = 1;  // 16-byte vectors of the larger copy, items of the more numerous
-    char *at = (char *)ws;
+    char *at = (char *)pads;
     auto copy = [&](const void *&src, int64_t &s_in, int64_t &s_out, int64_t &ld, int64_t rows, int64_t cols,
                     int64_t rows_p, int64_t dst_ld, int64_t items, size_t bytes) {
         pad.side[sides++] = PadSide{(const uint16_t *)src, s_in, s_out, ld, (uint16_t *)at, (uint32_t)rows,
@@ -1852,7 +1853,7 @@ it_status launch_ragged(it_context *ctx, bool ta, bool tb, GemmArgs a, const Rag
         const dim3 grid((unsigned)std::min<int64_t>(cdiv(most, 256), 8192), (unsigned)items_most, (unsigned)sides);
         hipLaunchKernelGGL(pad_bf16, grid, dim3(256), 0, ctx->stream, pad);
     }
-    a.partial = (float *)at;
+    a.partial = (float *)part;
     a.K = r.kp;
     a.a_vec_ok = a.b_vec_ok = a.c_vec_ok = 1;  // C: 4-column vectors of any alignment
     a.tiles_m = (int)cdiv(a.M, r.plan.bm);
@@ -1940,11 +1941,12 @@ it_status launch_gemm(it_context *ctx, it_dtype dtype_in, bool transA, bool tran
     double t_plan = 0.0;
     Plan plan = choose_plan(a, bf16, cus, transA, transB, &t_plan);
     if (Ragged r; bf16 && plan_ragged(a, cus, transA, transB, plan, t_plan, r)) {
-        const size_t bytes = r.bytes_a + r.bytes_b + r.bytes_part;
-        void *ws = nullptr;
+        const size_t bytes = r.bytes_a + r.bytes_b;
+        void *pads = nullptr, *part = nullptr;
         if (a.batch * r.plan.splits <= 65535) {
-            if (bytes == 0 || ensure_scratch(ctx, bytes, &ws) == IT_OK)
-                return launch_ragged(ctx, transA, transB, a, r, ws, profile_tag);
+            if ((bytes == 0 || ensure_pad_scratch(ctx, bytes, &pads) == IT_OK) &&
+                (r.bytes_part == 0 || ensure_scratch(ctx, r.bytes_part, &part) == IT_OK))
+                return launch_ragged(ctx, transA, transB, a, r, pads, part, profile_tag);
             clear_error();  // no scratch (a capture may not allocate): the plain tiles
         }
     }

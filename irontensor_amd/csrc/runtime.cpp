@@ -88,6 +88,10 @@ it_status ensure_attn_scratch(it_context *ctx, size_t bytes, void **out) {
     return grow(ctx, ctx->attn_scratch[ctx->cur], ctx->attn_scratch_bytes[ctx->cur], bytes, out);
 }
 
+it_status ensure_pad_scratch(it_context *ctx, size_t bytes, void **out) {
+    return grow(ctx, ctx->pad_scratch[ctx->cur], ctx->pad_scratch_bytes[ctx->cur], bytes, out);
+}
+
 it_status ensure_counters(it_context *ctx, int **out) {
     int *&f = ctx->counters[ctx->cur];
     if (!f) {
@@ -234,6 +238,7 @@ it_status it_shutdown(it_context *ctx) {
     for (int i = 0; i < 2; ++i) {
         if (ctx->scratch[i]) (void)hipFree(ctx->scratch[i]);
         if (ctx->attn_scratch[i]) (void)hipFree(ctx->attn_scratch[i]);
+        if (ctx->pad_scratch[i]) (void)hipFree(ctx->pad_scratch[i]);
         if (ctx->counters[i]) (void)hipFree(ctx->counters[i]);
     }
     (void)hipEventDestroy(ctx->fork_ev);
@@ -304,7 +309,7 @@ size_t it_mem_allocated(it_context *ctx) { return ctx ? ctx->bytes_live : 0; }
 size_t it_mem_scratch(it_context *ctx) {
     if (!ctx) return 0;
     size_t total = 0;
-    for (int i = 0; i < 2; ++i) total += ctx->scratch_bytes[i] + ctx->attn_scratch_bytes[i];
+    for (int i = 0; i < 2; ++i) total += ctx->scratch_bytes[i] + ctx->attn_scratch_bytes[i] + ctx->pad_scratch_bytes[i];
     for (auto &r : ctx->retired) total += r.second;
     return total;
 }
@@ -314,6 +319,13 @@ it_status it_empty_cache(it_context *ctx) {
     if (const it_status st_ = it::sync_all(ctx); st_ != IT_OK) return st_;
     for (auto &kv : ctx->cache) IT_HIP_TRY(hipFree(kv.second));
     ctx->cache.clear();
+    // A live graph may have been captured with the padded copies' addresses.
+    if (ctx->graphs.empty())
+        for (int i = 0; i < 2; ++i) {
+            if (ctx->pad_scratch[i]) IT_HIP_TRY(hipFree(ctx->pad_scratch[i]));
+            ctx->pad_scratch[i] = nullptr;
+            ctx->pad_scratch_bytes[i] = 0;
+        }
     return IT_OK;
 }
 

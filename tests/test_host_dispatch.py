@@ -114,3 +114,24 @@ got = keys(lambda: gemm(1, 0, 0, 1000, 1000, 4096, X.ptr, X.ptr, X.ptr, ldb=1 <<
 print(got)
 assert '_edge' not in got[0], got
 """)
+
+
+def test_padded_copies_are_given_back(fake):
+    """it_empty_cache frees the scratch of a ragged BF16 product's padded copies; while a graph is alive, which
+    may hold its address, it stays, and later products take it again."""
+    _run(fake, """
+A, B, Cc = buf(8001 * 4001 // 2 + 1), buf(4001 * 8003 // 2 + 1), buf(8001 * 8003)
+f = lambda: gemm(1, 0, 1, 8001, 8003, 4001, A.ptr, B.ptr, Cc.ptr)
+scratch = lambda: ctx.lib.it_mem_scratch(ctx.handle)
+before = scratch()
+assert '_dtl_edge' in keys(f)[0] and scratch() - before > 100e6
+assert ctx.lib.it_empty_cache(ctx.handle) == 0 and scratch() == before
+assert '_dtl_edge' in keys(f)[0] and scratch() - before > 100e6
+g = C.c_void_p()
+assert ctx.lib.it_capture_begin(ctx.handle) == 0 and f() == 0
+assert 'pad_bf16' in ' '.join(launches())
+assert ctx.lib.it_capture_end(ctx.handle, C.byref(g)) == 0
+assert ctx.lib.it_empty_cache(ctx.handle) == 0 and scratch() - before > 100e6
+assert ctx.lib.it_graph_destroy(g) == 0
+assert ctx.lib.it_empty_cache(ctx.handle) == 0 and scratch() == before
+""")
