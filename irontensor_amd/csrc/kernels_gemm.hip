@@ -1797,6 +1797,7 @@ bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &p
         e.a_vec_ok = e.b_vec_ok = 1;
         double t = 0.0;
         Plan pl = choose_plan(e, true, cus, ta, tb, &t);
+        if (plain.bm == 256 && plain.splits > 1) pl = Plan{256, 256, plain.splits, 0};  // as its price is compared
         if (pl.k_per_split <= 0) pl.k_per_split = cdiv(cdiv(e.K, pl.splits), 128) * 128;
         e.k_per_split = pl.k_per_split;
         bool dtl = pl.bm == 256 ? dtl_applicable(ta, tb, e, pl.bn) : pl.bm == 128 && dtl128_applicable(ta, tb, e);

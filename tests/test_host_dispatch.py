@@ -94,17 +94,6 @@ assert '_dtl_edge' in got[0], got
 """)
 
 
-def test_ragged_products_run_the_plan_that_was_priced(fake):
-    """A long ragged k whose plain plan is 256 x 256 tiles with split K: the edge tiles take the plan their
-    price is for, here one round of 256 x 128 tiles."""
-    _run(fake, """
-X = buf(1 << 25)
-got = keys(lambda: gemm(1, 1, 0, 1928, 2872, 1936, X.ptr, X.ptr, X.ptr))
-print(got)
-assert '_256x128_dtl_edge|' in got[0] and got[0].endswith(' s1'), got
-""")
-
-
 def test_operands_beyond_the_edge_tiles_offsets(fake):
     """A ragged product over a B whose k rows span more than 2 GiB a split has no edge-tile plan and stays on
     the plain tiles (launched on nothing here: the buffer is not that large)."""
