@@ -1894,6 +1894,9 @@ it_status launch_ragged(it_context *ctx, bool ta, bool tb, GemmArgs a, const Rag
 
 }  // namespace
 
+// Profiler keys of FP32 products on the FP32 units (those on the BF16 terms have the same keys without).
+constexpr const char *UNITS_TAG = "units:";
+
 it_status launch_splitk_reduce(hipStream_t s, const GemmArgs &a) {
     const int64_t total = a.batch * a.M * a.N;
     if (a.N % 4 == 0) {
@@ -2015,11 +2018,11 @@ it_status launch_gemm(it_context *ctx, it_dtype dtype_in, bool transA, bool tran
     hipEvent_t ev = nullptr;
     if (ctx->profiling) {
         char buf[192];
-        std::snprintf(buf, sizeof(buf), "gemm_%s_%c%c_%dx%d%s%s%s%s|%s[%lld,%lld,%lld]x%lld s%d",
+        std::snprintf(buf, sizeof(buf), "gemm_%s_%c%c_%dx%d%s%s%s%s|%s%s[%lld,%lld,%lld]x%lld s%d",
                       bf16 ? "bf16" : "f32", transA ? 'T' : 'N', transB ? 'T' : 'N', cfg.bm, cfg.bn,
                       dtl ? "_dtl" : "",
                       a.dual ? "_swiglu" : "", a.causal || a.kmode ? "_causal" : "", a.a_kscale ? "_rmsnorm" : a.xent_stats ? "_xent" : "",
-                      profile_tag ? profile_tag : "", (long long)a.M, (long long)a.N,
+                      bf16 ? "" : UNITS_TAG, profile_tag ? profile_tag : "", (long long)a.M, (long long)a.N,
                       (long long)a.K, (long long)a.batch, splits);
         key = buf;
         profile_begin(ctx, key, &ev);
@@ -2181,7 +2184,7 @@ bool launch_f32_group(it_context *ctx, bool ta, bool tb, GemmArgs *args, int cou
     std::string key;
     hipEvent_t ev = nullptr;
     if (ctx->profiling) {
-        key = std::string("gemm_f32_") + (ta ? 'T' : 'N') + (tb ? 'T' : 'N') + "_64x64_group|" + (tag ? tag : "");
+        key = std::string("gemm_f32_") + (ta ? 'T' : 'N') + (tb ? 'T' : 'N') + "_64x64_group|" + UNITS_TAG + (tag ? tag : "");
         for (int i = 0; i < count; ++i)
             key += (i ? "+[" : "[") + std::to_string(args[i].M) + "," + std::to_string(args[i].N) + "," +
                    std::to_string(args[i].K) + "]";

@@ -12,7 +12,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from irontensor_amd import _lib, synth
+from irontensor_amd import _lib, profiler, synth
 from tests.numerics import op
 
 pytestmark = pytest.mark.gpu
@@ -163,3 +163,49 @@ def test_infinities_in_every_wave(it, ta, tb, m, n, k):
     assert np.array_equal(got[rows], np.where(vb[cols] > 0, np.inf, -np.inf).astype(np.float32))
     rest = np.delete(np.arange(m), rows)
     _check(got[rest], np.ascontiguousarray(va[rest]), np.ascontiguousarray(vb), 0, 0, k)
+
+
+def _keys(it, fn):
+    ctx = it.Context.global_()
+    profiler.reset(ctx)
+    profiler.enable(ctx)
+    assert fn() == 0
+    keys = list(profiler.stats(ctx))
+    profiler.enable(ctx, False)
+    return keys
+
+
+@pytest.mark.parametrize("tile,splits,ta,tb,m,n,k", [
+    ("256x128", 1, 0, 0, 1621, 2489, 506), ("256x128", 1, 0, 1, 2177, 1803, 490), ("256x128", 8, 0, 0, 837, 971, 3202),
+    ("256x128", 2, 0, 1, 1127, 2749, 485), ("128x128", 1, 1, 1, 1207, 2861, 162), ("128x128", 2, 1, 0, 1537, 2166, 658),
+    ("128x128", 2, 0, 0, 1335, 2718, 828), ("128x128", 1, 0, 1, 2072, 2982, 27), ("128x128", 6, 0, 1, 772, 1345, 1666),
+    ("64x64", 1, 1, 0, 291, 246, 21), ("64x64", 3, 0, 0, 2117, 242, 730), ("64x64", 5, 0, 1, 149, 1887, 2467),
+    ("64x64", 8, 1, 0, 307, 220, 1007), ("64x64", 12, 1, 1, 655, 37, 1435), ("64x64", 1, 0, 1, 1470, 390, 17),
+    ("64x32", 1, 0, 0, 28, 594, 22), ("64x32", 3, 1, 1, 62, 455, 318), ("64x32", 12, 0, 1, 212, 126, 1830),
+    ("64x32", 4, 0, 0, 26, 194, 398), ("64x32", 24, 1, 0, 96, 35, 2973)])
+def test_every_tile_at_its_edges(it, tile, splits, ta, tb, m, n, k):
+    """Each tile shape and layout at sizes it does not divide, operands and output at odd columns of wider
+    buffers whose other elements are NaN (the output's: untouched). Gaussian data against float64: every
+    element within the bound, and the whole within 4e-7, where losing one of the 2^-16 term products
+    (each operand's terms are 2^-9 / sqrt(3) of the one before in the mean) would show 7e-7."""
+    a, b = _operands(41, m, n, k, ta, tb)
+    ctx = it.Context.global_()
+
+    def wide(x, fill):
+        w = np.full((x.shape[0] + 2, x.shape[1] + 7), fill, np.float32)
+        w[1:-1, 3:-4] = x
+        return it.Tensor.from_f32_slice(w, list(w.shape)), w.shape[1]
+
+    (A, lda), (B, ldb) = wide(a, np.nan), wide(b, np.nan)
+    Cw, ldc = wide(np.zeros((m, n), np.float32), 7.0)
+    ptr = lambda t, ld: C.c_void_p(t.ptr + 4 * (ld + 3))
+    keys = _keys(it, lambda: ctx.lib.it_gemm(ctx.handle, 0, 0, ta, tb, m, n, k, 1.0, ptr(A, lda), lda, 0, ptr(B, ldb), ldb,
+                                             0, 0.0, ptr(Cw, ldc), ldc, 0, 1, None))
+    assert keys == [f"gemm_f32_{'NT'[ta]}{'NT'[tb]}_{tile}|[{m},{n},{k}]x1 s{splits}"], keys
+    got = Cw.numpy()
+    y = got[1:-1, 3:-4].astype(np.float64)
+    _check(y, a, b, ta, tb, k)
+    exact = op(a, ta).astype(np.float64) @ op(b, tb).astype(np.float64)
+    assert np.linalg.norm(y - exact) <= 4e-7 * np.linalg.norm(exact)
+    got[1:-1, 3:-4] = 7.0
+    assert np.all(got == 7.0)

@@ -11,7 +11,8 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from irontensor_amd import _lib, synth
+from irontensor_amd import _lib, profiler, synth
+from tests.numerics import op
 
 pytestmark = pytest.mark.gpu
 
@@ -90,3 +91,75 @@ def test_cross_entropy_operand(it, units, tokens, vocab, h):
         A, B = np.ascontiguousarray(A), B[:, fine].astype(np.float64)
         n = A.shape[1]
         assert np.all(np.abs(got[:, fine] - A @ B) <= ((n + 2) * 2.0 ** -24 + 3e-6) * (np.abs(A) @ np.abs(B)))
+
+
+def _keys(it, fn):
+    ctx = it.Context.global_()
+    profiler.reset(ctx)
+    profiler.enable(ctx)
+    assert fn() == 0
+    keys = list(profiler.stats(ctx))
+    profiler.enable(ctx, False)
+    return keys
+
+
+@pytest.mark.parametrize("tile,ta,tb,m,n,k", [
+    ("256x128", 0, 0, 4096, 256, 16384), ("256x128", 0, 1, 4096, 256, 16384), ("128x128", 0, 1, 2279, 2554, 22),
+    ("128x128", 1, 0, 2356, 1812, 32), ("128x128", 0, 0, 2462, 2470, 17), ("128x128", 1, 1, 2021, 2978, 39),
+    ("64x64", 0, 1, 4096, 768, 256), ("64x64", 1, 0, 307, 220, 1007), ("64x64", 0, 0, 2225, 47, 491),
+    ("64x64", 1, 1, 1354, 515, 19), ("64x64", 0, 1, 129, 2868, 2781), ("64x64", 0, 0, 932, 44, 1592),
+    ("64x32", 0, 0, 4096, 256, 1376), ("64x32", 0, 1, 4096, 256, 688), ("64x32", 0, 1, 4000, 250, 700),
+    ("64x32", 1, 0, 4000, 250, 700), ("64x32", 0, 0, 1000, 90, 300), ("64x32", 1, 1, 609, 128, 1079),
+    ("64x32", 1, 0, 288, 28, 2208)])
+def test_every_tile_exact(it, tile, ta, tb, m, n, k):
+    """Every tile, whole and at sizes it does not divide (descriptor, masked and bounds-checked loads), with
+    alpha, beta and a bias: exact on small integers, whose sums are integers below 2^24."""
+    a = synth.small_ints(51, (k, m) if ta else (m, k), -3, 3)
+    b = synth.small_ints(52, (n, k) if tb else (k, n), -3, 3)
+    bias, c0 = synth.small_ints(53, (n,), -4, 4), synth.small_ints(54, (m, n), -4, 4)
+    T = it.Tensor.from_f32_slice
+    A, B, out, Bias = T(a, list(a.shape)), T(b, list(b.shape)), T(c0, [m, n]), T(bias, [n])
+    epi = _lib.Epilogue(flags=_lib.IT_EPI_BIAS | _lib.IT_EPI_F32_UNITS, bias=Bias.ptr)
+    keys = _keys(it, lambda: A.ctx.lib.it_gemm(A.ctx.handle, 0, 0, ta, tb, m, n, k, 2.0, C.c_void_p(A.ptr), a.shape[1], 0,
+                                               C.c_void_p(B.ptr), b.shape[1], 0, 3.0, C.c_void_p(out.ptr), n, 0, 1,
+                                               C.byref(epi)))
+    assert len(keys) == 1 and keys[0].startswith(f"gemm_f32_{'NT'[ta]}{'NT'[tb]}_{tile}|units:"), keys
+    ref = op(a, ta).astype(np.float64) @ op(b, tb).astype(np.float64)
+    assert np.array_equal(out.numpy(), (2 * ref + 3 * c0 + bias).astype(np.float32))
+
+
+@pytest.mark.parametrize("bt,m,n,k,shared", [(3, 65, 40, 96, False), (5, 200, 130, 37, True), (2, 300, 300, 128, False)])
+def test_batches_and_causal_outputs(it, bt, m, n, k, shared):
+    """Strided and shared operands of a batch, plain and with the causal mask (-inf above the diagonal)."""
+    a, b = synth.small_ints(61, (bt, m, k), -3, 3), synth.small_ints(62, (1 if shared else bt, n, k), -3, 3)
+    A, B = it.Tensor.from_f32_slice(a, list(a.shape)), it.Tensor.from_f32_slice(b, list(b.shape))
+    exact = np.matmul(a.astype(np.float64), np.swapaxes(b.astype(np.float64), 1, 2))
+    above = np.triu(np.ones((m, n), bool), 1)
+    for causal in (0, _lib.IT_EPI_CAUSAL):
+        out = it.Tensor.empty([bt, m, n])
+        epi = _lib.Epilogue(flags=_lib.IT_EPI_F32_UNITS | causal)
+        keys = _keys(it, lambda: A.ctx.lib.it_gemm(A.ctx.handle, 0, 0, 0, 1, m, n, k, 1.0, C.c_void_p(A.ptr), k, m * k,
+                                                   C.c_void_p(B.ptr), k, 0 if shared else n * k, 0.0, C.c_void_p(out.ptr), n,
+                                                   m * n, bt, C.byref(epi)))
+        assert "|units:" in keys[0], keys
+        want = np.where(above, -np.inf, exact) if causal else exact
+        assert np.array_equal(out.numpy(), want.astype(np.float32))
+
+
+@pytest.mark.parametrize("dims,k", [([(1376, 256), (256, 688), (768, 256), (256, 256)], 4096),
+                                    ([(100, 300), (301, 500), (65, 64)], 3001), ([(128, 128), (130, 132)], 100)])
+def test_group_exact(it, dims, k):
+    """Weight gradients as one grouped launch on the FP32 units, whole and ragged."""
+    T = it.Tensor.from_f32_slice
+    data = [(synth.small_ints(71 + i, (k, m), -2, 2), synth.small_ints(81 + i, (k, n), -2, 2)) for i, (m, n) in enumerate(dims)]
+    ops = [(T(x, list(x.shape)), T(y, list(y.shape)), it.Tensor.empty([m, n])) for (x, y), (m, n) in zip(data, dims)]
+    epi = _lib.Epilogue(flags=_lib.IT_EPI_F32_UNITS)
+    calls = (_lib.GemmCall * len(dims))(*[
+        _lib.GemmCall(1, 0, m, n, k, 1.0, x.ptr, m, 0, y.ptr, n, 0, 0.0, o.ptr, n, 0, 1, C.pointer(epi))
+        for (x, y, o), (m, n) in zip(ops, dims)])
+    ctx = ops[0][0].ctx
+    keys = _keys(it, lambda: ctx.lib.it_gemm_group(ctx.handle, 0, 0, len(dims), calls))
+    print(f"[units group] {keys}", flush=True)
+    assert len(keys) == 1 and keys[0].startswith("gemm_f32_TN_64x64_group|units:"), keys
+    for (x, y), (_, _, o) in zip(data, ops):
+        assert np.array_equal(o.numpy(), (x.T.astype(np.float64) @ y.astype(np.float64)).astype(np.float32))

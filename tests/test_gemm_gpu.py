@@ -790,7 +790,7 @@ def test_bf16_128_tile_split_k_exact(it, m, n, k):
 @pytest.mark.parametrize("tb", [False, True])
 def test_f32_256_tile_exact(it, tb):
     """FP32 data gradients of the LM-head shape ([4096, 256, 16384], X.W and X.W^T) run on the
-    256 x 128 FP32 tile with split K (one block per CU): exact on small integers against a float64
+    256 x 128 tile of the BF16 terms with split K (one block per CU): exact on small integers against a float64
     product (every partial sum is an integer below 2^24), with alpha and a bias in the epilogue
     that follows the split-K reduction."""
     from irontensor_amd import profiler
@@ -816,8 +816,8 @@ def test_f32_256_tile_exact(it, tb):
                                        (4000, 250, 700, "NT"), (4000, 250, 700, "TN"), (1000, 90, 300, "NN")])
 def test_f32_64x32_tile_exact(it, m, n, k, lay):
     """FP32 GEMMs the planner runs on the 64 x 32 tile (two blocks per CU where 64 x 64 tiles leave
-    one): the TINY step's [4096, 256, K] data gradients and projections, and ragged shapes (masked or
-    bounds-checked loads at every edge). Exact on small integers against a float64 product, with
+    one): the TINY step's [4096, 256, K] data gradients and projections, and ragged shapes (the terms'
+    descriptor loads; tests/test_f32_units_gpu.py takes the FP32 units' tile). Exact on small integers against a float64 product, with
     alpha and a bias in the epilogue; the TINY shapes' plan key names the tile."""
     from irontensor_amd import profiler
     ta, tb = lay[0] == "T", lay[1] == "T"
