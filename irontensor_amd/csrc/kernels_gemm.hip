@@ -1806,16 +1806,17 @@ bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &p
         e.a_vec_ok = e.b_vec_ok = 1;
         double t = 0.0;
         Plan pl = choose_plan(e, true, cus, ta, tb, &t);
-        const bool as_plain = plain.bm == 256 && plain.splits > 1;
-        if (as_plain) {
-            // The plain plan's tile and splits, at the price they have as edge tiles. The model would rather have
+        if (plain.bm == 256 && plain.splits > 1) {
+            // The plain plan's tile and splits, at the price they have as edge tiles (partial sums at 5 TB/s: with
+            // that [1000, 2800, 8010] of a transposed A takes them, 80.2 us against 82.1 on 128 x 128 tiles, and
+            // [2577, 1298, 11675] those, 123.9 against 134.2). The model would rather have
             // fewer splits of smaller tiles: over 60 random shapes 13 change then, 4.5% faster in the geometric
             // mean but up to 9% slower ([2504, 2496, 11856] 170.4 -> 185.9 us).
             pl = Plan{256, 256, plain.splits, 0};
             const int64_t kps = cdiv(cdiv(r.kp, pl.splits), 128) * 128, splits = cdiv(r.kp, kps);
             const int64_t blocks = cdiv(a.M, 256) * cdiv(a.N, 256) * a.batch * splits;
             t = cdiv(blocks, cus) * (3e-6 + dtl_block_time(kps, 256, ta)) +
-                2.0 * splits * a.M * a.N * a.batch * 4.0 / 4e12 + 4e-6;
+                2.0 * splits * a.M * a.N * a.batch * 4.0 / 5e12 + 4e-6;
         }
         if (pl.k_per_split <= 0) pl.k_per_split = cdiv(cdiv(e.K, pl.splits), 128) * 128;
         e.k_per_split = pl.k_per_split;
@@ -1830,7 +1831,6 @@ bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &p
             best = t;
             r.plan = pl;
         }
-        if (as_plain && dtl && pl.bm == 256) break;
     }
     if (best >= 1e30) return false;  // no direct-to-LDS tile spans the operands in place
     r.bytes_part = r.plan.splits > 1 ? (size_t)r.plan.splits * a.batch * a.M * a.N * sizeof(float) : 0;
