@@ -36,8 +36,9 @@ import numpy as np
 ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
-# FP32 products run as six BF16 products each (the FP32 units reach 157.3).
-PEAK_TFLOPS = {"f32": 2500.0 / 6, "bf16": 2500.0}
+# FP32 products run as six BF16 products each ("f32"); those that ask for the FP32 units, such as the
+# training step's, on units of 157.3.
+PEAK_TFLOPS = {"f32": 2500.0 / 6, "f32_units": 157.3, "bf16": 2500.0}
 PEAK_HBM_GBS = 8000.0
 
 
@@ -139,7 +140,7 @@ def extra_config1(it, timer) -> dict:
     ms = time_gemm(it, timer, x, w, y, False, True, 50)
     tf = 2 * 4096 * 768 * 256 / (ms * 1e-3) / 1e12
     return {"config1_fp32_qkv_4096x768x256_NT": {"ms": round(ms, 5), "tflops": round(tf, 2),
-                                                 "frac_fp32_peak": round(tf / PEAK_TFLOPS["f32"], 4)}}
+                                                 "frac_f32_terms_peak": round(tf / PEAK_TFLOPS["f32"], 4)}}
 
 
 def extra_attention(it, timer) -> dict:
@@ -901,7 +902,8 @@ def main() -> int:
             "tied_lm_head": False, "batch": 16, "seq": 256, "gflop_per_step": round(total_flops / 1e9, 2),
             "gemm_launches": len(step.launches),
             "execution": "hipGraph replay on one stream; each layer's weight gradients as one grouped launch",
-            "frac_fp32_mfma_peak": round(total_flops / (ms_per_step * 1e-3) / 1e12 / PEAK_TFLOPS["f32"], 4),
+            "frac_f32_terms_peak": round(total_flops / (ms_per_step * 1e-3) / 1e12 / PEAK_TFLOPS["f32"], 4),
+            "frac_fp32_mfma_peak": round(total_flops / (ms_per_step * 1e-3) / 1e12 / PEAK_TFLOPS["f32_units"], 4),
             "ms_per_step_side_stream": round(ms_side, 4),
             "tflops_side_stream": round(total_flops / (ms_side * 1e-3) / 1e12, 3),
             "attention_gflop_dense_equiv": round(attn_flops / 1e9, 2),

@@ -123,9 +123,12 @@ it_status it_event_destroy(it_event *ev);
 #define IT_EPI_ROPE 0x8u        /* rotary embedding of columns n < rope_cols (src/ops/rope.rs:22) */
 #define IT_EPI_SWIGLU_BWD 0x10u /* SwiGLU backward of the product (src/ops/backward/elementwise.rs:149) */
 #define IT_EPI_XENT_A 0x20u     /* A = logits read as their cross-entropy gradient (src/ops/backward/loss.rs:248) */
-#define IT_EPI_F32_UNITS 0x40u  /* FP32 inputs: sums on the FP32 matrix units in k order (combines with any flag;
-                                   without it FP32 products run as BF16 terms, which is faster and nearer to
-                                   the exact sums, and rounds differently) */
+#define IT_EPI_F32_UNITS 0x40u  /* FP32 inputs: sums on the FP32 matrix units in k order (combines with any flag) */
+/* Without IT_EPI_F32_UNITS an FP32 product of more than 16 rows runs as BF16 terms that carry all 24 bits of
+ * every operand: on average faster and nearer to the exact sums than the FP32 units, and it rounds
+ * differently. Where results are not finite, operands exceed 2^112 or sums 2^96, those tiles are summed on the
+ * FP32 units, at about half their speed. Splits of k need scratch: a capture takes the best plan that the
+ * scratch of earlier calls allows, so a product captured before it has run outside may round differently. */
 
 typedef struct it_epilogue {
     uint32_t flags;

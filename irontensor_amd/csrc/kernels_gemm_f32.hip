@@ -1,8 +1,8 @@
 // FP32 GEMMs on the BF16 matrix units: every operand element is split into three BF16 terms on its way
 // into LDS (split_bf16x3: 24 significand bits), and a product takes the six term products down to
 // 2^-16 of the whole, accumulated in FP32. The FP32 units reach 157 TFLOP/s; six BF16 products per
-// FP32 product 417 at the nominal BF16 rate and 228 at the rate the largest BF16 products reach on
-// this card.
+// FP32 product 417 at the nominal BF16 rate and 204 at the rate that a large BF16 product reaches on
+// this card (1223).
 //
 // Design (per k-tile of 32):
 //   * global -> registers with 128-bit buffer loads (k-contiguous operands: 4 k of a row; mn-contiguous
@@ -10,7 +10,7 @@
 //     way). A descriptor ends at the operand's last element and its range check, dword by dword,
 //     supplies the zeros past it; the loads need no more than an element's alignment. So every size
 //     and leading dimension runs the same loop (a 1000 x 300 x 701 layer forward and backward: 53 us
-//     with the FP32-unit kernels, whose loads go element by element there, 46 here);
+//     with the FP32-unit kernels, whose loads go element by element there, 41 here);
 //   * split, then three LDS planes [rows][32 k] of 64-byte rows; a lane's fragment of one term is one
 //     128-bit LDS read;
 //   * v_mfma_f32_16x16x32_bf16 blocks (the 32x32x16 form measured 2-6% slower in these tiles);
@@ -777,8 +777,8 @@ void any_alignment(GemmArgs &a) { a.c_vec_ok = a.c_vec_ok || !a.out_bf16; }
 }  // namespace
 
 bool f32_terms_applicable(const GemmArgs &a, bool ta, bool tb) {
-    // A few rows wait on latency, not on the matrix units: M = 1, N = 768, K = 256 takes 6.7 us here
-    // and 6.0 on the FP32 units' 64 x 32 tile, which loads two k-tiles ahead.
+    // A few rows wait on latency, not on the matrix units: M = 1, N = 768, K = 256 takes 0.7 us more here
+    // than on the FP32 units' 64 x 32 tile, which loads two k-tiles ahead.
     // (X.W^T there goes to gemv_nt where its rows are whole 16-byte chunks.)
     // More rows stay here for their precision also where the FP32 units are faster, which they are in
     // products of few k-tiles (a k-tile's split sits between its load and its products): K = 256 FP32
