@@ -1765,10 +1765,14 @@ double dtl_block_time(int64_t k, int bn, bool ta) {
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
-// False where the product is another kernel's or the ordinary plan is priced lower. That plan's price is
-// corrected for its loads at such sizes: measured 57 TFLOP/s element by element (1999 x 3001 x 1237) and
-// 265 with masked vectors (2000 x 3000 x 1240) where the model says about 250 and 420; the copies cost
-// 3 us and their traffic at 2.5 TB/s.
+// False where the product is another kernel's or the ordinary plan is priced lower. Both prices are corrected
+// for such sizes, fitted on 160 random ragged shapes (64 to 8192 rows and columns, 64 to 11008 k, a fifth of
+// them batches), each timed on the plain and on the edge tiles: the plain tiles with masked vectors take
+// twice their price less 3 us (256 x 256: four times), with element loads three times and 7 us; the edge
+// tiles 0.9 of theirs and 5 us, with copies 9 us and the copies' traffic more. The picks take 0.4% longer than
+// the faster of the two. With factors from two nearby shapes (1.6 and 4.0, 3 us for copies) they took 7.3%:
+// small products of whole vectors went to the edge tiles and slowed down ([448, 1776, 64] of a transposed A
+// 7.0 -> 12.7 us, [7840, 392, 152] 10.9 -> 16.5).
 // plain, t_plain: the ordinary plan and its estimate.
 bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &plain, double t_plain, Ragged &r) {
     constexpr int bk = ET<uint16_t>::BK;
@@ -1781,7 +1785,8 @@ bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &p
     if (plain.bm == 256 ? dtl_applicable(ta, tb, d, plain.bn) : plain.bm == 128 && dtl128_applicable(ta, tb, d))
         return false;
     const bool vectors = vectors_exact<uint16_t>(a, ta, tb);
-    if (!tiles_exact(d, plain.bm, plain.bn, bk)) t_plain *= vectors && plain.bm != 256 ? 1.6 : 4.0;
+    if (!tiles_exact(d, plain.bm, plain.bn, bk))
+        t_plain = vectors ? (plain.bm != 256 ? 2.0 : 4.0) * t_plain - 3e-6 : 3.0 * t_plain + 7e-6;
 
     r.kp = cdiv(a.K, 128) * 128;
     r.copy_a = !a.a_vec_ok || r.kp != a.K;
@@ -1794,7 +1799,7 @@ bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &p
     r.items_b = a.sB_in == 0 && a.sB_out == 0 ? 1 : a.batch;
     r.bytes_a = r.copy_a ? align256((size_t)r.items_a * r.rows_a * r.ld_a * 2) : 0;
     r.bytes_b = r.copy_b ? align256((size_t)r.items_b * r.rows_b * r.ld_b * 2) : 0;
-    const double copies = ((r.copy_a || r.copy_b) ? 3e-6 : 0.0) + 2.0 * (r.bytes_a + r.bytes_b) / 2.5e12;
+    const double extra = 5e-6 + ((r.copy_a || r.copy_b) ? 9e-6 : 0.0) + 2.0 * (r.bytes_a + r.bytes_b) / 10e12;
     double best = 1e30;
     for (const int unit : {256, 128}) {  // whole tiles of this unit cover the product
         GemmArgs e = a;
@@ -1834,7 +1839,7 @@ bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &p
     }
     if (best >= 1e30) return false;  // no direct-to-LDS tile spans the operands in place
     r.bytes_part = r.plan.splits > 1 ? (size_t)r.plan.splits * a.batch * a.M * a.N * sizeof(float) : 0;
-    return best + copies < t_plain && r.bytes_a + r.bytes_b <= (size_t(1) << 30);
+    return 0.9 * best + extra < t_plain && r.bytes_a + r.bytes_b <= (size_t(1) << 30);
 }
 
 it_status launch_ragged(it_context *ctx, bool ta, bool tb, GemmArgs a, const Ragged &r, void *pads, void *part,
