@@ -43,6 +43,7 @@ def test_exact_in_every_layout(it, m, n, k, ta, tb):
 
 
 def test_batched_bias_alpha_beta_and_bf16_output(it):
+    """A ragged batch that is priced onto the plain tiles (test_batched_epilogues_on_edge_tiles has the others)."""
     bt, m, n, k = 3, 301, 517, 200
     a, b = synth.small_ints(1, (bt, m, k), -3, 3), synth.small_ints(2, (n, k), -3, 3)
     bias, c0 = synth.small_ints(3, (n,), -4, 4), synth.small_ints(4, (bt, m, n), -4, 4)

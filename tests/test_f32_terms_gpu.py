@@ -44,8 +44,8 @@ def test_layouts_and_edges(it, m, n, k, ta, tb):
 
 
 @pytest.mark.parametrize("ta,tb", LAYOUTS)
-@pytest.mark.parametrize("tile_n,m,n,k", [(256, 512, 384, 4096), (128, 640, 1152, 96), (64, 192, 200, 40)])
-def test_strided_unaligned_operands(it, tile_n, m, n, k, ta, tb):
+@pytest.mark.parametrize("m,n,k", [(512, 384, 4096), (640, 1152, 96), (192, 200, 40)])
+def test_strided_unaligned_operands(it, m, n, k, ta, tb):
     """Rows at any element alignment: operands and output inside wider buffers, starting at odd columns,
     whose surrounding elements are NaN (they may be read past K and past an edge, never used) or must
     stay untouched."""
@@ -100,9 +100,8 @@ def test_nonfinite_and_extreme_operands(it, m, n, k, ta, tb):
         A64, B64 = va.astype(np.float64), vb.astype(np.float64)
         exact, size = A64 @ B64, np.abs(A64) @ np.abs(B64)
         err = np.abs(got.astype(np.float64) - exact)[fine]
-        # BF16's smallest step is 2^-133: an element's terms miss it by half of that at most.
-        tiny = 2.0 ** -134 * np.broadcast_to(np.abs(B64).sum(0), exact.shape)[fine] + 2.0 ** -140
-    assert np.all(err <= (k / 8 + 16) * 2.0 ** -23 * size[fine] + tiny)
+    # (sums of subnormal results round to FP32's smallest step, 2^-149, once per product)
+    assert np.all(err <= (k / 8 + 16) * 2.0 ** -23 * size[fine] + 2.0 ** -140)
 
 
 @pytest.mark.parametrize("rows,h,f", [(65, 33, 49), (200, 256, 688), (1024, 128, 2048)])
