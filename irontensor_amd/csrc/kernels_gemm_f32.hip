@@ -706,7 +706,7 @@ void launch_plain(int bm, int bn, const GemmArgs &a, dim3 grid, hipStream_t s) {
 // share of the CU's time) and of one that has it alone, a round's launch, prologue and epilogue, and what a
 // transposed A costs a k-tile (64-byte pieces of its rows, which the 64 x 32 tile waits for). Fitted on
 // every tile and split count of 110 shapes, warm: the TINY step's, ragged ones, squares, and random ones
-// of 17 to 8192 rows and up to 16384 columns and 11008 k. The picks take 1.3% longer than the fastest
+// of 17 to 8192 rows and up to 16384 columns and 11008 k. The picks take 1.9% longer than the fastest
 // measured plans; the former constants, with powers of two as split counts, took 5.4%, up to 1.4x
 // ([701, 300, 1000] of a transposed A 19.7 us on 64 x 32 tiles, 14.8 on 64 x 64 with four splits).
 struct Tile {
@@ -715,7 +715,10 @@ struct Tile {
 };
 constexpr Tile T256{256, 128, 1, 2.08, 2.43, 15.4, 1.0}, T128{128, 128, 2, 1.36, 2.41, 12.6, 1.0},
     T64{64, 64, 3, 0.52, 0.69, 4.8, 1.0}, T6432{64, 32, 2, 0.307, 0.34, 4.9, 1.5};
-constexpr double PARTIAL_BW = 3.1e12, REDUCE = 1.6e-6;  // split-K partial sums out and back, the reduction
+// Split-K partial sums out and back, and the reduction's launch: 4 us, where device times alone gave 1.6, because
+// small products wait on the host, which a second launch keeps longer (a 112 x 96 x 514 layer, called from
+// Python, 32.5 us unsplit and 36.8 split; the 110 shapes take 0.6% more for it). A group adds in the kernel.
+constexpr double PARTIAL_BW = 3.1e12, REDUCE = 4e-6, GROUP_SUM = 1.6e-6;
 constexpr int SPLITS[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
 
 struct Plan {
@@ -902,7 +905,7 @@ bool launch_gemm_f32_group(it_context *ctx, bool ta, bool tb, const GemmArgs *ar
         }
         if (!ok) break;
         double t = group_time(blocks, ksteps, cus);
-        if (traffic > 0.0) t += traffic / PARTIAL_BW + REDUCE;  // the tiles' last blocks add the partial sums
+        if (traffic > 0.0) t += traffic / PARTIAL_BW + GROUP_SUM;  // the tiles' last blocks add the partial sums
         if (t < best_t) {
             best_t = t;
             best_s = s;
