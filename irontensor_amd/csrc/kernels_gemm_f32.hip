@@ -705,20 +705,26 @@ void launch_plain(int bm, int bn, const GemmArgs &a, dim3 grid, hipStream_t s) {
 // The tiles as the planner prices them, in microseconds: a k-tile of a block that shares its CU (its
 // share of the CU's time) and of one that has it alone, a round's launch, prologue and epilogue, and what a
 // transposed A costs a k-tile (64-byte pieces of its rows, which the 64 x 32 tile waits for). Fitted on
-// every tile and split count of 110 shapes, warm: the TINY step's, ragged ones, squares, and random ones
-// of 17 to 8192 rows and up to 16384 columns and 11008 k. The picks take 1.9% longer than the fastest
-// measured plans; the former constants, with powers of two as split counts, took 5.4%, up to 1.4x
-// ([701, 300, 1000] of a transposed A 19.7 us on 64 x 32 tiles, 14.8 on 64 x 64 with four splits).
+// every tile and split count of 132 shapes, warm: the TINY step's, ragged ones, squares, layers of up to
+// 8192 rows, and random ones of 17 to 8192 rows and up to 16384 columns and 11008 k. The picks take 1.4%
+// longer than the fastest measured plans; the former constants, with powers of two as split counts, took
+// 5% and up to 1.4x ([701, 300, 1000] of a transposed A 19.7 us on 64 x 32 tiles, 14.8 on 64 x 64 with four
+// splits).
 struct Tile {
     int bm, bn, occ;  // occ: blocks a CU runs at once
     double shared, alone, round, ta;
 };
-constexpr Tile T256{256, 128, 1, 2.08, 2.43, 15.4, 1.0}, T128{128, 128, 2, 1.36, 2.41, 12.6, 1.0},
-    T64{64, 64, 3, 0.52, 0.69, 4.8, 1.0}, T6432{64, 32, 2, 0.307, 0.34, 4.9, 1.5};
+constexpr Tile T256{256, 128, 1, 1.97, 1.97, 14.4, 1.0}, T128{128, 128, 2, 1.05, 1.42, 12.3, 1.0},
+    T64{64, 64, 3, 0.55, 0.715, 2.8, 1.0}, T6432{64, 32, 2, 0.314, 0.332, 2.95, 1.51},
+    TGROUP{64, 64, 3, 0.50, 0.60, 3.0, 1.0};  // a group's 64 x 64 blocks, fitted on eleven groups
+// The SwiGLU form's epilogue weighs more on the wide tile's few blocks: [4096, 688, 256] takes 26.9 us on
+// 64 x 64 and 28.3 on 128 x 128, [8192, 688, 256] 46.4 and 42.1, [8192, 2816, 1024] 586 and 464. Over 35
+// shapes the picks take 0.2% longer than the faster tile.
+constexpr Tile T128_DUAL{128, 128, 2, 1.05, 1.42, 14.5, 1.0};
 // Split-K partial sums out and back, and the reduction's launch: 4 us, where device times alone gave 1.6, because
 // small products wait on the host, which a second launch keeps longer (a 112 x 96 x 514 layer, called from
-// Python, 32.5 us unsplit and 36.8 split; the 110 shapes take 0.6% more for it). A group adds in the kernel.
-constexpr double PARTIAL_BW = 3.1e12, REDUCE = 4e-6, GROUP_SUM = 1.6e-6;
+// Python, 32.5 us unsplit and 36.8 split). A group adds in the kernel.
+constexpr double PARTIAL_BW = 5.4e12, REDUCE = 4e-6, GROUP_BW = 3.1e12, GROUP_SUM = 1.6e-6;
 constexpr int SPLITS[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
 
 struct Plan {
@@ -726,21 +732,15 @@ struct Plan {
     int64_t k_per_split;
 };
 
-// One launch of `blocks` blocks of ksteps k-tiles, in seconds.
+// One launch of `blocks` blocks of ksteps k-tiles, in seconds: whole rounds of the blocks that a CU runs at
+// once, and a last one that costs what the blocks it gives a CU take alone ([3333, 3333, 2222] on 128 x 128
+// tiles: 512 blocks and 217 more, 300 us, against 338 for two nearly full rounds of 256 x 128; the TINY
+// layer's group: five splits, 980 blocks, 65.5 us, four, 784 in one round and 16 more, 75.6).
 double launch_time(const Tile &t, bool ta, int64_t blocks, int64_t ksteps, int64_t cus) {
-    const int64_t per_cu = cdiv(blocks, cus), conc = std::min<int64_t>(per_cu, t.occ);
-    return 1e-6 * cdiv(per_cu, t.occ) * (t.round + (ta ? t.ta : 1.0) * ksteps * std::max(conc * t.shared, t.alone));
-}
-
-// A group's launch of 64 x 64 blocks, in seconds: its rounds overlap less evenly than one product's, so a
-// last round that a few blocks fill costs what they take alone. Fitted on eleven groups of two to four
-// products: the split counts it picks take 0.1% longer than the fastest (the TINY layer's four weight
-// gradients: five splits, 980 blocks, 65.5 us; four, 784 blocks in one round and 16 more, 75.6).
-double group_time(int64_t blocks, int64_t ksteps, int64_t cus) {
-    constexpr Tile t{64, 64, 3, 0.50, 0.60, 3.0, 1.0};
     const int64_t full = blocks / (t.occ * cus), rest = cdiv(blocks % (t.occ * cus), cus);
-    return 1e-6 * (full * (t.round + ksteps * std::max(t.occ * t.shared, t.alone)) +
-                   (rest ? t.round + ksteps * std::max(rest * t.shared, t.alone) : 0.0));
+    const double ktiles = (ta ? t.ta : 1.0) * ksteps;
+    return 1e-6 * (full * (t.round + ktiles * std::max(t.occ * t.shared, t.alone)) +
+                   (rest ? t.round + ktiles * std::max(rest * t.shared, t.alone) : 0.0));
 }
 
 // Picks the tile and the split count, lowest price first. Near ties (3%) keep the earlier
@@ -753,7 +753,7 @@ Plan choose_plan(const GemmArgs &a, int64_t cus, bool ta, double *est) {
     Plan best{64, a.dual ? 32 : 64, 1, kall};
     double best_t = 1e30;
     int64_t best_blocks = 0;
-    for (const Tile &tile : {T256, T128, T64, T6432}) {
+    for (const Tile &tile : {T256, a.dual ? T128_DUAL : T128, T64, T6432}) {
         if (tile.bm != tile.bn && (!plain || a.xent_stats)) continue;
         if (tile.bm == 256 && (ta || a.swiglu_bwd || a.rope_table)) continue;
         const int bn = a.dual ? tile.bn / 2 : tile.bn;
@@ -904,8 +904,8 @@ bool launch_gemm_f32_group(it_context *ctx, bool ta, bool tb, const GemmArgs *ar
             if (splits > 1) traffic += 2.0 * splits * a.M * a.N * 4.0;
         }
         if (!ok) break;
-        double t = group_time(blocks, ksteps, cus);
-        if (traffic > 0.0) t += traffic / PARTIAL_BW + GROUP_SUM;  // the tiles' last blocks add the partial sums
+        double t = launch_time(TGROUP, ta, blocks, ksteps, cus);
+        if (traffic > 0.0) t += traffic / GROUP_BW + GROUP_SUM;  // the tiles' last blocks add the partial sums
         if (t < best_t) {
             best_t = t;
             best_s = s;

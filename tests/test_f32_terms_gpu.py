@@ -175,9 +175,9 @@ def _keys(it, fn):
 
 
 @pytest.mark.parametrize("tile,splits,ta,tb,m,n,k", [
-    ("256x128", 1, 0, 0, 1621, 2489, 506), ("256x128", 1, 0, 1, 2177, 1803, 490), ("256x128", 8, 0, 0, 837, 971, 3202),
-    ("256x128", 2, 0, 1, 2277, 1357, 571), ("128x128", 1, 1, 1, 1207, 2861, 162), ("128x128", 3, 1, 0, 1766, 1293, 1585),
-    ("128x128", 2, 0, 0, 1335, 2718, 828), ("128x128", 1, 0, 1, 2072, 2982, 27), ("128x128", 6, 0, 1, 772, 1345, 1666),
+    ("256x128", 1, 0, 0, 1510, 2863, 1283), ("256x128", 1, 0, 1, 1410, 2803, 1241), ("256x128", 8, 0, 0, 837, 971, 3202),
+    ("256x128", 2, 0, 1, 2281, 1353, 1104), ("128x128", 1, 1, 1, 1985, 1681, 226), ("128x128", 3, 1, 0, 1766, 1293, 1585),
+    ("128x128", 3, 0, 0, 1221, 1000, 1087), ("128x128", 1, 0, 1, 1173, 2713, 283), ("128x128", 6, 0, 1, 772, 1345, 1666),
     ("64x64", 1, 1, 0, 291, 246, 21), ("64x64", 3, 0, 0, 2154, 226, 1390), ("64x64", 5, 0, 1, 149, 1887, 2467),
     ("64x64", 8, 1, 0, 307, 220, 1007), ("64x64", 12, 1, 1, 655, 37, 1435), ("64x64", 1, 0, 1, 1470, 390, 17),
     ("64x32", 1, 0, 0, 28, 594, 22), ("64x32", 5, 1, 1, 31, 355, 557), ("64x32", 12, 0, 1, 212, 126, 1830),
