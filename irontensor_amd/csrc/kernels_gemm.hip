@@ -1770,9 +1770,9 @@ size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 // them batches), each timed on the plain and on the edge tiles: the plain tiles with masked vectors take
 // twice their price less 3 us (256 x 256: four times), with element loads three times and 7 us; the edge
 // tiles 0.9 of theirs and 5 us, with copies 9 us and the copies' traffic more. The picks take 0.4% longer than
-// the faster of the two, on 160 other shapes 0.7%, on 120 read in place 0.5%. With factors from two nearby shapes (1.6 and 4.0, 3 us for copies) they took 6 to
-// 8.5%: small products of whole vectors went to the edge tiles and slowed down ([448, 1776, 64] of a transposed A
-// 7.0 -> 12.7 us, [7840, 392, 152] 10.9 -> 16.5).
+// the faster of the two, on 160 other shapes 0.7%, on 120 read in place 0.5%. With factors from two nearby
+// shapes (1.6 and 4.0, 3 us for copies) they took 6 to 8.5%: small products of whole vectors went to the edge
+// tiles and slowed down ([448, 1776, 64] of a transposed A 7.0 -> 12.7 us, [7840, 392, 152] 10.9 -> 16.5).
 // plain, t_plain: the ordinary plan and its estimate.
 bool plan_ragged(const GemmArgs &a, int64_t cus, bool ta, bool tb, const Plan &plain, double t_plain, Ragged &r) {
     constexpr int bk = ET<uint16_t>::BK;
