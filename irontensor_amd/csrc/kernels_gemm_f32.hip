@@ -793,8 +793,8 @@ bool f32_terms_applicable(const GemmArgs &a, bool ta, bool tb) {
     // More rows stay here for their precision also where the FP32 units are faster, which they are in
     // products of few k-tiles (a k-tile's split sits between its load and its products): K = 256 FP32
     // units 2.9e-7 from 64 bits and 9.9 us against 0.9e-7 and 11.6 ([4096, 256, 256], X.W), 512^3 9.6
-    // against 11.9. Over 110 shapes (choose_plan) the terms are 1.10x as fast, from 0.66x ([192, 176, 160] of
-    // a transposed A) to 2.1x; callers that would rather have the time ask for the units (IT_EPI_F32_UNITS).
+    // against 11.9. Over 127 of choose_plan's shapes the terms are 1.20x as fast, from 0.65x ([192, 176, 160]
+    // of a transposed A) to 3.0x; callers that would rather have the time ask for the units (IT_EPI_F32_UNITS).
     return a.M > 16 && !a.f32_units && !a.a_kscale && spans_fit(a, ta, tb);
 }
 
